@@ -32,25 +32,38 @@
 //     slices are spread over the XCDs (work-groups are dispatched to the 8
 //     XCDs round-robin), so each XCD's L2 caches one slice of the hot
 //     feature rows and holds SL times as many of them;
+//   * a wave reads its rows 64 at a time, one per lane: offsets, original id,
+//     divisor and the way the row reaches C go into an LDS window, so the
+//     rows that follow cost no memory round trip of their own.  Column
+//     indices and values are fetched with coalesced streaming loads into an
+//     LDS stage of 256 consecutive nonzeros that all chunks read, long and
+//     short (one round trip per 256 nonzeros instead of one per 64 of a long
+//     row and one per group of short ones).  What bounds short rows is this
+//     chain of dependent round trips, not bandwidth: with offsets and
+//     indices read group by group, the 2^18-row R-MAT at K = 75 took 310 us
+//     (206 now), the 2^21-row one at K = 96 1,817 us (1,515), the 4,096-row
+//     uniform graph at K = 32 14.7 us (9.9).  Keeping the window in LDS also
+//     frees registers: 78 instead of 87-89 VGPRs at K = 32 to 128;
 //   * short rows run row-per-slot, RU rows per slot at a time, each row
 //     summed sequentially in CSR order (bit-identical to the reference's
-//     per-work-item loop);
+//     per-work-item loop); a group of no more rows than slots takes RU
+//     consecutive nonzeros of its row per round trip instead;
+//   * a stretch of rows to be stored as zeros is stored in one go: group by
+//     group, a wave's 164 such rows of the 2^18-row R-MAT at K = 75 took
+//     74 us, longer than all other waves (half of that graph's rows);
 //   * a long chunk runs on all slots at once, UL nonzeros in flight per
 //     slot, followed by a shuffle reduction across slots;
-//   * the occupancy variant (O6) keeps UL <= 2, which lets slots of 4 to 16
-//     lanes fit 80 VGPRs: 6 waves per SIMD instead of 5, for graphs of
-//     short rows, where waves in flight set the speed;
+//   * the occupancy variant (O6) keeps UL <= 2 and asks for 6 waves per SIMD
+//     in slots of 4 to 16 lanes (75 VGPRs; the standard kernel's 78 give 6
+//     too), for graphs of short rows, where waves in flight set the speed
+//     (16M-row mesh, runs by output row, 1 task per wave: 939 us standard,
+//     923 us O6);
 //   * column phases (PH, csrc/col_phases.hip): the launch is repeated once
 //     per band of columns (c mod P) over a copy of the CSR sorted by band
 //     within each row, so that the feature rows all waves gather at a time
 //     fit the caches; on a chain of tasks each run owns whole rows, stored
 //     in the first phase and added to without atomics in the others;
-//   * column indices and values are fetched with coalesced streaming loads:
-//     64 at a time for a long chunk, handed to the slots with cross-lane
-//     shuffles; for a group of short rows, the group's whole contiguous
-//     range (up to 256 nonzeros) at once, into a per-wave LDS window, so no
-//     row waits on an index load before its feature-row loads.  C is written
-//     with streaming stores.
+//   * C is written with streaming stores.
 // Split rows are cleared by zero_split_rows before the main kernel: a row
 // that a segment leaves open is cleared by the task whose chunk of it starts
 // at nonzero 0.
@@ -69,6 +82,8 @@ namespace {
 constexpr int kWaves = 1;
 constexpr int kBlock = 64 * kWaves;
 constexpr int kAuxBlock = 256;
+// Column indices and values of one stage of the aggregation kernel.
+constexpr int kStage = 256;
 // A launch holds fewer than 2^32 work-items.
 constexpr long long kMaxGridBlocks = (1ll << 32) / kBlock - 8;
 
@@ -237,11 +252,14 @@ __device__ __forceinline__ void write_row(float* p, typename VecT<VEC>::T v, int
         vatomic_add(p, v);
 }
 
-__device__ __forceinline__ int wave_max(int v)
+// Orders a wave's LDS accesses before and after an exchange between its
+// lanes: the hardware keeps them in order, the fences keep the compiler from
+// moving them across.
+__device__ __forceinline__ void wave_lds_fence()
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off));
-    return v;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Nonzero range of row r inside task (rs, re, fo, ln), with the reference's
@@ -414,16 +432,16 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
     constexpr int UL = O6 ? cmin(cmin(U, G), 2) : cmin(U, G);
     constexpr int STEP = NS * UL;                  // nonzeros per wave step (<= 64)
     constexpr int kLong = GROUP > 2 ? GROUP : 2;   // chunk length that runs on all slots
-    // A short-row group holds at most GROUP * (kLong - 1) nonzeros.  When
-    // that can exceed 64, a group's nonzeros (up to kStage, the group is cut
-    // there) go through a per-wave LDS window; otherwise through one
-    // 64-entry register window.  Either way no row waits on a column-index
-    // load before its feature-row loads.
-    constexpr int kMaxGroupNnz = GROUP * (kLong - 1);
-    constexpr int kStage = kMaxGroupNnz > 64 ? cmin(kMaxGroupNnz, 256) : 0;
-    constexpr int kWin = kStage > 0 ? kStage : 64;  // nonzeros of one group
-    __shared__ int s_col[kWaves * (kStage > 0 ? kStage : 1)];
-    __shared__ float s_val[kWaves * (kStage > 0 ? kStage : 1)];
+    // The wave's row window (up to 64 rows: where each row's chunk starts and
+    // ends, its original id, its divisor and how it reaches C) and its stage
+    // (up to kStage consecutive column indices and values).
+    __shared__ int s_beg[kWaves * 64];
+    __shared__ int s_end[kWaves * 64];
+    __shared__ int s_out[kWaves * 64];
+    __shared__ float s_deg[kWaves * 64];
+    __shared__ int s_how[kWaves * 64];
+    __shared__ int s_col[kWaves * kStage];
+    __shared__ float s_val[kWaves * kStage];
 
     const int lane = threadIdx.x & 63;
     const int slot = lane / G;
@@ -444,8 +462,13 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
         ph = __builtin_amdgcn_readfirstlane(status[1]) != seq;
         if (!ph && !first) return;
     }
-    int* __restrict__ wcol = s_col + wv * (kStage > 0 ? kStage : 1);
-    float* __restrict__ wval = s_val + wv * (kStage > 0 ? kStage : 1);
+    int* const wbeg = s_beg + wv * 64;
+    int* const wend = s_end + wv * 64;
+    int* const wout = s_out + wv * 64;
+    float* const wdeg = s_deg + wv * 64;
+    int* const whow = s_how + wv * 64;
+    int* const wcol = s_col + wv * kStage;
+    float* const wval = s_val + wv * kStage;
     // run_order (optional) is a permutation of [0, n_runs): runs execute in
     // that order instead of task order.
     const long long run = run_order ? static_cast<long long>(run_order[pos]) : pos;
@@ -473,287 +496,326 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
         const bool bph = PH && ph && banded;
         const int rlo = max(rs, 0);
         const int rhi = min(re, n_rows);
+        // The staged nonzeros: [st0, st0 + stn) of cx / vx.
+        int st0 = 0;
+        int stn = 0;
+        // Stages the nonzeros from `from` up to `to`, at most kStage of them:
+        // all loads first, then the LDS writes, one memory round trip.
+        auto stage = [&](const int from, const int to) {
+            const int n = min(kStage, to - from);
+            constexpr int NT = kStage / 64;
+            int lc[NT];
+            float lv[NT];
+            const int lane = fresh(threadIdx.x & 63);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const int i = lane + 64 * t;
+                lc[t] = i < n ? __builtin_nontemporal_load(cx + from + i) : 0;
+                lv[t] = i < n ? __builtin_nontemporal_load(vx + from + i) : 0.0f;
+                if constexpr (HN)
+                    if (i < n) lc[t] = with_hint(lc[t], hints, from + i);
+            }
+            wave_lds_fence();
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const int i = lane + 64 * t;
+                if (i < n) {
+                    wcol[i] = lc[t];
+                    wval[i] = lv[t];
+                }
+            }
+            wave_lds_fence();
+            st0 = from;
+            stn = n;
+        };
         for (int pass = 0; pass < npass; ++pass) {
             const int fl = pass * G * R + sub;  // first vector element of this lane
-            int r = rlo;
-            while (r < rhi) {
-                // With groups of 32 or more short rows, each lane of the first
-                // GROUP reads its row's chunk before the long/short decision,
-                // which takes lane 0's (row r): the group's offsets and row
-                // r's arrive in one memory round trip (measured on the 16M-row
-                // mesh: 1.7-3.5% faster).  Smaller groups read row r's chunk
-                // alone first (faster on R-MAT, whose runs hold long rows).
-                constexpr bool kEarly = GROUP >= 32;
-                const int lane_g = fresh(threadIdx.x & 63);
-                const int rr = r + lane_g;
-                const bool mine = lane_g < GROUP && rr < rhi;
-                Chunk my = {0, 0, 0, 0};
-                Chunk c0;
-                if constexpr (kEarly) {
-                    if (mine) my = task_chunk<PH>(rp, rr, rs, re, fo, ln, nnz, bph, pb, pe);
-                    c0.base = __builtin_amdgcn_readfirstlane(my.base);
-                    c0.b = __builtin_amdgcn_readfirstlane(my.b);
-                    c0.e = __builtin_amdgcn_readfirstlane(my.e);
-                    c0.d = __builtin_amdgcn_readfirstlane(my.d);
-                    if constexpr (PH) c0.own = __builtin_amdgcn_readfirstlane(my.own);
-                } else {
-                    c0 = task_chunk<PH>(rp, r, rs, re, fo, ln, nnz, bph, pb, pe);
-                }
-                const int len0 = c0.e - c0.b;
-                if (len0 >= kLong) {
-                    // ---------------- long chunk: all slots on one row
-                    V acc[R];
-#pragma unroll
-                    for (int q = 0; q < R; ++q) acc[q] = vzero<VEC>();
-                    // (an unsigned step: a chunk may end within 64 of 2^31)
-                    for (unsigned uw = c0.b; uw < static_cast<unsigned>(c0.e); uw += 64u) {
-                        const int w0 = static_cast<int>(uw);
-                        const int wn = min(64, c0.e - w0);
-                        const int lane = fresh(threadIdx.x & 63);
-                        int colw = 0;
-                        float valw = 0.0f;
-                        if (lane < wn) {
-                            colw = __builtin_nontemporal_load(cx + c0.base + w0 + lane);
-                            valw = __builtin_nontemporal_load(vx + c0.base + w0 + lane);
-                            if constexpr (HN) colw = with_hint(colw, hints, c0.base + w0 + lane);
-                        }
-                        for (int k0 = 0; k0 < wn; k0 += STEP) {
-                            int cc[UL];
-                            float a[UL];
-                            bool ok[UL];
-                            bool cold[UL];
-                            const int sl = fresh(slot);
-#pragma unroll
-                            for (int u = 0; u < UL; ++u) {
-                                const int jj = k0 + u * NS + sl;
-                                cc[u] = __shfl(colw, jj & 63);
-                                a[u] = __shfl(valw, jj & 63);
-                                cold[u] = HN && cc[u] < 0;
-                                if constexpr (HN) cc[u] &= 0x7fffffff;
-                                ok[u] = jj < wn;
-                                if (ok[u] && static_cast<unsigned long long>(cc[u]) >=
-                                                 static_cast<unsigned long long>(h_rows)) {
-                                    ok[u] = false;
-                                    bad |= 1;
-                                }
-                            }
-                            V h[UL][R];
-#pragma unroll
-                            for (int u = 0; u < UL; ++u) {
-                                const float* hrow = Hs + static_cast<size_t>(cc[u]) * ld;
-#pragma unroll
-                                for (int q = 0; q < R; ++q) {
-                                    const int f = fl + G * q;
-                                    if constexpr (HN)
-                                        h[u][q] = (ok[u] && f < F)
-                                                      ? gather_hinted(hrsrc,
-                                                                      static_cast<unsigned>(cc[u]) * ld * 4u +
-                                                                          slice_bytes + f * 16u,
-                                                                      cold[u])
-                                                      : vzero<VEC>();
-                                    else
-                                        h[u][q] = (ok[u] && f < F) ? vload<VEC>(hrow + f * VEC)
-                                                                   : vzero<VEC>();
-                                }
-                            }
-#pragma unroll
-                            for (int u = 0; u < UL; ++u) {
-                                if (ok[u]) {
-#pragma unroll
-                                    for (int q = 0; q < R; ++q) acc[q] = vfma(a[u], h[u][q], acc[q]);
-                                }
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int off = G; off < 64; off <<= 1) {
-#pragma unroll
-                        for (int q = 0; q < R; ++q) acc[q] = acc[q] + vshfl_xor(acc[q], off);
-                    }
-                    const int o = origin[r];
-                    if (static_cast<unsigned>(o) >= static_cast<unsigned>(n_rows)) {
-                        bad |= 2;
-                    } else if (slot == 0) {
-                        float* crow = Cs + static_cast<size_t>(o) * ld;
-                        const float fd = static_cast<float>(c0.d);
-                        const int how = write_mode<PH>(bph, first, c0);
-#pragma unroll
-                        for (int q = 0; q < R; ++q) {
-                            const int f = fl + G * q;
-                            if (f < F) write_row<VEC>(crow + f * VEC, vdiv(acc[q], fd), how);
-                        }
-                    }
-                    ++r;
-                    continue;
-                }
-
-                // ---------------- short rows: one row per slot, RU rows per slot
-                const int lane = lane_g;
-                if constexpr (!kEarly) {
-                    if (mine) my = task_chunk<PH>(rp, rr, rs, re, fo, ln, nnz, bph, pb, pe);
-                }
-                const int mylen = my.e - my.b;
-                // The group: the leading rows that are short, start where the
-                // previous row's chunk ends (always, for a non-decreasing
-                // row_ptr) and end within kWin nonzeros of the group's start.
-                // The first row always qualifies (its chunk is shorter than
-                // kLong <= kWin), so every group makes progress, and the
-                // group's nonzeros are the contiguous range [gs, gs + gn).
-                const int mys = my.base + my.b;
-                const int mye = my.base + my.e;
-                const int gs = c0.base + c0.b;
-                const int prev_end = __shfl_up(mye, 1);
-                const bool fits = mine && mylen < kLong && (lane == 0 || mys == prev_end) &&
-                                  mye - gs <= kWin;
-                const unsigned long long stop = __ballot(!fits);
-                int cnt = min(GROUP, rhi - r);
-                if (stop) cnt = min(cnt, static_cast<int>(__ffsll(static_cast<long long>(stop))) - 1);
-                const int myo = (mine && lane < cnt) ? origin[rr] : 0;
-                const int ge = __shfl(mye, cnt - 1);
-                const int gn = (gs >= 0 && static_cast<long long>(ge) <= nnz) ? ge - gs : 0;
-                int colw = 0;
-                float valw = 0.0f;
-                if constexpr (kStage > 0) {
-                    // The previous group's reads of this wave's window are done
-                    // (wave-ordered LDS); the fences keep the compiler from
-                    // moving accesses across the exchange.
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    // All loads first, then the LDS writes: one memory round trip.
-                    constexpr int NT = (kStage + 63) / 64;
-                    int lc[NT];
-                    float lv[NT];
-#pragma unroll
-                    for (int t = 0; t < NT; ++t) {
-                        const int i = lane + 64 * t;
-                        lc[t] = i < gn ? __builtin_nontemporal_load(cx + gs + i) : 0;
-                        lv[t] = i < gn ? __builtin_nontemporal_load(vx + gs + i) : 0.0f;
-                        if constexpr (HN)
-                            if (i < gn) lc[t] = with_hint(lc[t], hints, gs + i);
-                    }
-#pragma unroll
-                    for (int t = 0; t < NT; ++t) {
-                        const int i = lane + 64 * t;
-                        if (i < gn) {
-                            wcol[i] = lc[t];
-                            wval[i] = lv[t];
-                        }
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                } else if (lane < gn) {
-                    colw = __builtin_nontemporal_load(cx + gs + lane);
-                    valw = __builtin_nontemporal_load(vx + gs + lane);
-                    if constexpr (HN) colw = with_hint(colw, hints, gs + lane);
-                }
-                V acc[RU][R];
-                int pos[RU];
-                int len[RU];
-                int maxlen = 0;
-#pragma unroll
-                for (int u = 0; u < RU; ++u) {
-                    const int gi = u * NS + fresh(slot);
-                    pos[u] = __shfl(mys - gs, gi);  // window position of the chunk
-                    len[u] = __shfl(mylen, gi);
-                    if (gi >= cnt) len[u] = 0;
-                    maxlen = max(maxlen, len[u]);
-#pragma unroll
-                    for (int q = 0; q < R; ++q) acc[u][q] = vzero<VEC>();
-                }
-                const int jmax = wave_max(maxlen);
-                for (int j = 0; j < jmax; ++j) {
-                    int cc[RU];
-                    float a[RU];
-                    bool ok[RU];
-                    bool cold[RU];
-#pragma unroll
-                    for (int u = 0; u < RU; ++u) {
-                        ok[u] = j < len[u];
-                        const int src = pos[u] + j;  // in [0, gn) whenever ok[u]
-                        if constexpr (kStage > 0) {
-                            cc[u] = wcol[ok[u] ? src : 0];
-                            a[u] = wval[ok[u] ? src : 0];
-                        } else {
-                            cc[u] = __shfl(colw, src & 63);
-                            a[u] = __shfl(valw, src & 63);
-                        }
-                        cold[u] = HN && cc[u] < 0;
-                        if constexpr (HN) cc[u] &= 0x7fffffff;
-                        if (ok[u] && static_cast<unsigned long long>(cc[u]) >=
-                                         static_cast<unsigned long long>(h_rows)) {
-                            ok[u] = false;
-                            bad |= 1;
-                        }
-                    }
-                    V h[RU][R];
-#pragma unroll
-                    for (int u = 0; u < RU; ++u) {
-                        const float* hrow = Hs + static_cast<size_t>(cc[u]) * ld;
-#pragma unroll
-                        for (int q = 0; q < R; ++q) {
-                            const int f = fl + G * q;
-                            if constexpr (HN)
-                                h[u][q] = (ok[u] && f < F)
-                                              ? gather_hinted(hrsrc,
-                                                              static_cast<unsigned>(cc[u]) * ld * 4u +
-                                                                  slice_bytes + f * 16u,
-                                                              cold[u])
-                                              : vzero<VEC>();
-                            else
-                                h[u][q] = (ok[u] && f < F) ? vload<VEC>(hrow + f * VEC) : vzero<VEC>();
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < RU; ++u) {
-                        if (ok[u]) {
-#pragma unroll
-                            for (int q = 0; q < R; ++q) acc[u][q] = vfma(a[u], h[u][q], acc[u][q]);
-                        }
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < RU; ++u) {
-                    const int gi = u * NS + fresh(slot);
-                    const int o = __shfl(myo, gi);
-                    Chunk cu;
-                    cu.d = __shfl(my.d, gi);
-                    cu.b = __shfl(my.b, gi);
-                    cu.e = __shfl(my.e, gi);
-                    if constexpr (PH) cu.own = __shfl(my.own, gi);
-                    if (gi < cnt) {
-                        if (cu.d < 0) {
+            for (int r0 = rlo, wcnt; r0 < rhi; r0 += wcnt) {
+                // ---------------- the row window: one row per lane
+                wcnt = min(64, rhi - r0);
+                unsigned long long longm;  // rows that run on all slots
+                unsigned long long live;   // rows with anything to do
+                unsigned long long some;   // rows with nonzeros
+                int last_end;
+                {
+                    const int lane = fresh(threadIdx.x & 63);
+                    Chunk c = {0, 0, 0, 0, 0};
+                    int o = 0;
+                    int how = 3;
+                    if (lane < wcnt) {
+                        o = origin[r0 + lane];
+                        c = task_chunk<PH>(rp, r0 + lane, rs, re, fo, ln, nnz, bph, pb, pe);
+                        if (c.d < 0) {
                             bad |= 4;
-                            continue;
-                        }
-                        if (static_cast<unsigned>(o) >= static_cast<unsigned>(n_rows)) {
+                            c.base = 0;  // malformed offsets: an empty chunk
+                        } else if (static_cast<unsigned>(o) >= static_cast<unsigned>(n_rows)) {
                             bad |= 2;
-                            continue;
+                        } else if (c.d == 0) {
+                            how = (first && write_empty) ? 0 : 3;
+                        } else if (c.e > c.b || (bph && first && c.own)) {
+                            // (an owned row with no nonzero in the first
+                            // phase is stored as zeros all the same)
+                            how = write_mode<PH>(bph, first, c);
                         }
-                        float* crow = Cs + static_cast<size_t>(o) * ld;
-                        if (cu.d == 0) {
-                            if (first && write_empty) {
+                    }
+                    const int cb = c.base + c.b;
+                    const int ce = c.base + c.e;
+                    longm = __ballot(c.e - c.b >= kLong);
+                    some = __ballot(c.e > c.b);
+                    live = some | __ballot(how != 3);
+                    last_end = __builtin_amdgcn_readlane(ce, wcnt - 1);
+                    wave_lds_fence();
+                    wbeg[lane] = cb;
+                    wend[lane] = ce;
+                    wout[lane] = o;
+                    wdeg[lane] = static_cast<float>(max(c.d, 1));
+                    whow[lane] = how;
+                    wave_lds_fence();
+                }
+                while (live) {
+                    const int w = __builtin_ctzll(live);
+                    if ((longm >> w) & 1ull) {
+                        // ---------------- long chunk: all slots on one row
+                        live &= live - 1;
+                        const int cb = __builtin_amdgcn_readfirstlane(wbeg[w]);
+                        const int ce = __builtin_amdgcn_readfirstlane(wend[w]);
+                        V acc[R];
 #pragma unroll
-                                for (int q = 0; q < R; ++q) {
-                                    const int f = fl + G * q;
-                                    if (f < F) vstore_nt<VEC>(crow + f * VEC, vzero<VEC>());
+                        for (int q = 0; q < R; ++q) acc[q] = vzero<VEC>();
+                        for (int at = cb; at < ce;) {
+                            // The part of the chunk that is staged: all that
+                            // is left of it, or a whole stage of its own.
+                            if (at < st0 || at - st0 >= stn ||
+                                (ce - st0 > stn && at != st0))
+                                stage(at, bph ? ce : max(last_end, ce));
+                            const int off = at - st0;
+                            const int wn = min(stn - off, ce - at);
+                            for (int k0 = 0; k0 < wn; k0 += STEP) {
+                                int cc[UL];
+                                float a[UL];
+                                bool ok[UL];
+                                bool cold[UL];
+                                const int sl = fresh(slot);
+#pragma unroll
+                                for (int u = 0; u < UL; ++u) {
+                                    const int jj = k0 + u * NS + sl;
+                                    ok[u] = jj < wn;
+                                    const int src = ok[u] ? off + jj : 0;
+                                    cc[u] = wcol[src];
+                                    a[u] = wval[src];
+                                    cold[u] = HN && cc[u] < 0;
+                                    if constexpr (HN) cc[u] &= 0x7fffffff;
+                                    if (ok[u] && static_cast<unsigned long long>(cc[u]) >=
+                                                     static_cast<unsigned long long>(h_rows)) {
+                                        ok[u] = false;
+                                        bad |= 1;
+                                    }
+                                }
+                                V h[UL][R];
+#pragma unroll
+                                for (int u = 0; u < UL; ++u) {
+                                    const float* hrow = Hs + static_cast<size_t>(cc[u]) * ld;
+#pragma unroll
+                                    for (int q = 0; q < R; ++q) {
+                                        const int f = fl + G * q;
+                                        if constexpr (HN)
+                                            h[u][q] = (ok[u] && f < F)
+                                                          ? gather_hinted(hrsrc,
+                                                                          static_cast<unsigned>(cc[u]) * ld * 4u +
+                                                                              slice_bytes + f * 16u,
+                                                                          cold[u])
+                                                          : vzero<VEC>();
+                                        else
+                                            h[u][q] = (ok[u] && f < F) ? vload<VEC>(hrow + f * VEC)
+                                                                       : vzero<VEC>();
+                                    }
+                                }
+#pragma unroll
+                                for (int u = 0; u < UL; ++u) {
+                                    if (ok[u]) {
+#pragma unroll
+                                        for (int q = 0; q < R; ++q)
+                                            acc[q] = vfma(a[u], h[u][q], acc[q]);
+                                    }
                                 }
                             }
-                        } else if (cu.e > cu.b || (bph && first && cu.own)) {
-                            // (an owned row with no nonzero in the first phase
-                            // is stored as zeros all the same)
-                            const float fd = static_cast<float>(cu.d);
-                            const int how = write_mode<PH>(bph, first, cu);
+                            at += wn;
+                        }
+#pragma unroll
+                        for (int off = G; off < 64; off <<= 1) {
+#pragma unroll
+                            for (int q = 0; q < R; ++q) acc[q] = acc[q] + vshfl_xor(acc[q], off);
+                        }
+                        const int how = __builtin_amdgcn_readfirstlane(whow[w]);
+                        if (how != 3 && slot == 0) {
+                            const int o = __builtin_amdgcn_readfirstlane(wout[w]);
+                            float* crow = Cs + static_cast<size_t>(o) * ld;
+                            const float fd = wdeg[w];
 #pragma unroll
                             for (int q = 0; q < R; ++q) {
                                 const int f = fl + G * q;
-                                if (f < F) write_row<VEC>(crow + f * VEC, vdiv(acc[u][q], fd), how);
+                                if (f < F) write_row<VEC>(crow + f * VEC, vdiv(acc[q], fd), how);
+                            }
+                        }
+                        continue;
+                    }
+
+                    if (!((some >> w) & 1ull)) {
+                        // ---------------- a stretch of rows to be stored as
+                        // zeros, NS * kZero at a time: nothing to wait for
+                        // but the row ids, read from LDS kZero at once.
+                        constexpr int kZero = 8;
+                        const unsigned long long other = ~(live & ~some) >> w;
+                        const int cz = other ? static_cast<int>(__builtin_ctzll(other)) : 64 - w;
+                        live = w + cz >= 64 ? 0ull : live & (~0ull << (w + cz));
+                        for (int i0 = 0; i0 < cz; i0 += NS * kZero) {
+                            int o[kZero];
+                            const int sl = i0 + fresh(slot);
+#pragma unroll
+                            for (int u = 0; u < kZero; ++u)
+                                o[u] = wout[w + min(u * NS + sl, cz - 1)];
+#pragma unroll
+                            for (int u = 0; u < kZero; ++u) {
+                                if (u * NS + sl < cz) {
+                                    float* crow = Cs + static_cast<size_t>(o[u]) * ld;
+#pragma unroll
+                                    for (int q = 0; q < R; ++q) {
+                                        const int f = fl + G * q;
+                                        if (f < F) vstore_nt<VEC>(crow + f * VEC, vzero<VEC>());
+                                    }
+                                }
+                            }
+                        }
+                        continue;
+                    }
+
+                    // ---------------- short rows: one row per slot, RU rows per slot.
+                    // The group: up to GROUP rows from row w on, to the next
+                    // long one, whose nonzeros are staged.  Row w is staged if
+                    // it is not yet (its chunk is shorter than kLong <=
+                    // kStage), so every group makes progress.
+                    const int after = wcnt - w;
+                    const unsigned long long nextl = longm >> w;
+                    const int upto = min(min(GROUP, after),
+                                         nextl ? static_cast<int>(__builtin_ctzll(nextl)) : 64);
+                    int cnt;
+                    {
+                        const int lane = fresh(threadIdx.x & 63);
+                        const int i = w + (lane < upto ? lane : 0);
+                        const int b = wbeg[i];
+                        const int e = wend[i];
+                        const int fb = __builtin_amdgcn_readfirstlane(b);
+                        const int fe = __builtin_amdgcn_readfirstlane(e);
+                        if (fb < st0 || fb - st0 >= stn || fe - st0 > stn)
+                            stage(fb, bph ? fe : max(last_end, fe));
+                        const bool fits = lane < upto &&
+                                          (e <= b || (b >= st0 && b - st0 < stn && e - st0 <= stn));
+                        const unsigned long long stop = __ballot(!fits);
+                        cnt = stop ? static_cast<int>(__builtin_ctzll(stop)) : 64;
+                    }
+                    live = w + cnt >= 64 ? 0ull : live & (~0ull << (w + cnt));
+                    V acc[RU][R];
+                    int pos[RU];
+                    int len[RU];
+                    int maxlen = 0;
+#pragma unroll
+                    for (int u = 0; u < RU; ++u) {
+                        const int gi = u * NS + fresh(slot);
+                        const int i = w + (gi < cnt ? gi : 0);
+                        pos[u] = wbeg[i];
+                        len[u] = gi < cnt ? wend[i] - pos[u] : 0;
+                        pos[u] -= st0;  // the chunk's place in the stage
+                        maxlen = max(maxlen, len[u]);
+#pragma unroll
+                        for (int q = 0; q < R; ++q) acc[u][q] = vzero<VEC>();
+                    }
+                    // One nonzero of each of the slot's RU rows at a time;
+                    // where the group has no more rows than slots, RU
+                    // consecutive nonzeros of its one row: as many loads in
+                    // flight, a RU-th of the round trips.
+                    const bool single = RU > 1 && cnt <= NS;
+                    const int jstep = single ? RU : 1;
+                    for (int j = 0; __ballot(j < maxlen) != 0ull; j += jstep) {
+                        int cc[RU];
+                        float a[RU];
+                        bool ok[RU];
+                        bool cold[RU];
+#pragma unroll
+                        for (int u = 0; u < RU; ++u) {
+                            const int ju = single ? j + u : j;
+                            ok[u] = ju < (single ? len[0] : len[u]);
+                            const int src = ok[u] ? (single ? pos[0] : pos[u]) + ju : 0;  // in [0, stn)
+                            cc[u] = wcol[src];
+                            a[u] = wval[src];
+                            cold[u] = HN && cc[u] < 0;
+                            if constexpr (HN) cc[u] &= 0x7fffffff;
+                            if (ok[u] && static_cast<unsigned long long>(cc[u]) >=
+                                             static_cast<unsigned long long>(h_rows)) {
+                                ok[u] = false;
+                                bad |= 1;
+                            }
+                        }
+                        V h[RU][R];
+#pragma unroll
+                        for (int u = 0; u < RU; ++u) {
+                            const float* hrow = Hs + static_cast<size_t>(cc[u]) * ld;
+#pragma unroll
+                            for (int q = 0; q < R; ++q) {
+                                const int f = fl + G * q;
+                                if constexpr (HN)
+                                    h[u][q] = (ok[u] && f < F)
+                                                  ? gather_hinted(hrsrc,
+                                                                  static_cast<unsigned>(cc[u]) * ld * 4u +
+                                                                      slice_bytes + f * 16u,
+                                                                  cold[u])
+                                                  : vzero<VEC>();
+                                else
+                                    h[u][q] = (ok[u] && f < F) ? vload<VEC>(hrow + f * VEC)
+                                                               : vzero<VEC>();
+                            }
+                        }
+                        if (single) {
+#pragma unroll
+                            for (int u = 0; u < RU; ++u) {
+                                if (ok[u]) {
+#pragma unroll
+                                    for (int q = 0; q < R; ++q) acc[0][q] = vfma(a[u], h[u][q], acc[0][q]);
+                                }
+                            }
+                        } else {
+#pragma unroll
+                            for (int u = 0; u < RU; ++u) {
+                                if (ok[u]) {
+#pragma unroll
+                                    for (int q = 0; q < R; ++q) acc[u][q] = vfma(a[u], h[u][q], acc[u][q]);
+                                }
+                            }
+                        }
+                    }
+                    int how[RU];
+                    int o[RU];
+                    float fd[RU];
+#pragma unroll
+                    for (int u = 0; u < RU; ++u) {
+                        const int gi = u * NS + fresh(slot);
+                        const int i = w + (gi < cnt ? gi : 0);
+                        how[u] = gi < cnt ? whow[i] : 3;
+                        o[u] = wout[i];
+                        fd[u] = wdeg[i];
+                    }
+#pragma unroll
+                    for (int u = 0; u < RU; ++u) {
+                        if (how[u] != 3) {
+                            float* crow = Cs + static_cast<size_t>(o[u]) * ld;
+#pragma unroll
+                            for (int q = 0; q < R; ++q) {
+                                const int f = fl + G * q;
+                                if (f < F)
+                                    write_row<VEC>(crow + f * VEC, vdiv(acc[u][q], fd[u]), how[u]);
                             }
                         }
                     }
                 }
-                r += cnt;
             }
         }
     };
@@ -1225,9 +1287,12 @@ void pick_tiling(int F, int SL, bool packed, bool wide, int* G_out, int* R_out)
 //     8.6 GB: K=128 2 slices 1.4% faster than 4, K=256 3.5% faster; K=512
 //     4 slices 2% faster than 2; K=192 2 slices 18% faster than 1);
 //   * tasks per wave M: the largest M that keeps at least 64 waves per CU
-//     (runs x slices) and at most ~256 rows per run (long runs of short rows
-//     serialise latency: the 16M-row mesh is 9% faster at 4 tasks per wave
-//     than at 16), clamped to [1, 64].
+//     (runs x slices) and at most ~64 rows per run, one row window: a second
+//     window is a second round trip to the offsets with nothing else in
+//     flight, and the last waves of the launch are longer (16M-row mesh:
+//     1,168 us at 1 task per wave, 1,176 at 2, 1,245 at 4, 1,273 at 7, where
+//     256 rows per run put it; 2^21-row R-MAT at K = 96: 1,487 us at 16,
+//     1,505 at 32), clamped to [1, 64].
 Plan make_plan(const cwlb_ctx* ctx, const SpmmArgs& a, bool per_task)
 {
     Plan p{};
@@ -1248,7 +1313,7 @@ Plan make_plan(const cwlb_ctx* ctx, const SpmmArgs& a, bool per_task)
         } else {
             const long long waves = static_cast<long long>(std::max(ctx->compute_units, 1)) * 64;
             const long long m_par = a.n_tasks * p.sl / waves;
-            const long long m_rows = a.n_rows > 0 ? 256 * a.n_tasks / a.n_rows : 64;
+            const long long m_rows = a.n_rows > 0 ? 64 * a.n_tasks / a.n_rows : 64;
             p.M = static_cast<int>(std::max<long long>(1, std::min({m_par, m_rows, 64ll})));
         }
     }
