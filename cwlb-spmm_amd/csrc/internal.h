@@ -54,6 +54,9 @@ struct cwlb_ctx {
     int order_M = 0;
     void* d_sort_temp = nullptr;
     size_t sort_temp_bytes = 0;
+    // Grow-only workspace of the GPU partition.
+    void* d_part = nullptr;
+    size_t part_bytes = 0;
     // Set when a launch under graph capture used d_run_order (resp.
     // d_hints): the graph keeps that address, so a later rebuild moves the
     // buffer to `retired` (freed by cwlb_ctx_destroy) and builds into a new

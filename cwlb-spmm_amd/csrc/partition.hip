@@ -10,18 +10,30 @@
 //   A(r)  at row r, the open task starts at row r, offset 0, load 0;
 //   B(r)  at long row r, the open task starts at row r, offset deg % S
 //         (the prefix went to the previous task), load 0.
-// From a fresh node the machine is deterministic up to the next fresh node.
-// So the partition is computed as
-//   1. part_transitions: every node simulates to its next node and counts
-//      the tasks it emits on the way (the host's double operations, in the
-//      host's order; this file is compiled without fp contraction);
-//   2. pointer doubling J_k = J_{k-1} o J_{k-1} until 2^k steps from A(0)
-//      reach the end;
-//   3. the chain from A(0) expanded by position in k rounds;
-//   4. an exclusive scan of the chain nodes' task counts;
-//   5. part_emit: each chain node simulates again and writes its tasks.
-// Node ids: A(r) = r for r in [0, n] (A(n) is the end), B(r) = n + 1 + c
-// where c is r's index among the long rows.
+// From a fresh node the machine is deterministic up to the next fresh node,
+// which lies at a later row (or is the B node of a later one).  The chain of
+// fresh nodes from A(0) is followed block by block of kRows rows:
+//   1. part_check: whether the offsets never decrease (then packs of short
+//      rows are found by binary search, partition_sim.h);
+//   2. part_blocks: every node of a block simulates to its next node and
+//      counts its tasks, then pointer doubling in LDS gives each node the
+//      first node outside the block and the tasks up to it.  A task covers
+//      fewer than max_scan rows, so a chain enters a block within its first
+//      max_scan + 1 rows: only those nodes' results are kept;
+//   3. part_groups: the same over groups of about sqrt(blocks) blocks, a
+//      thread per entry node hopping from block to block;
+//   4. part_walk: one thread hops from group to group, then a thread per
+//      group from block to block: every block's entry node and first task;
+//   5. part_emit: as part_blocks, but the doubling also marks the nodes on
+//      the chain from the block's entry node; each marked node simulates
+//      again and writes its tasks; rows of 64 segments or more are set aside;
+//   6. part_segments: a wave writes the tasks of such a row.
+// Nothing is written when the total exceeds the caller's buffer.  The host waits once, for the total and the status.  Measured on the
+// 4.2M-row R-MAT graph (1.08M tasks): 12.7 ms per call when the doubling ran
+// over all nodes of the graph in global memory (23 jump tables, 413 MB
+// allocated and freed by the call), 345 us now (part_emit 190, part_blocks 58,
+// part_walk 35, part_groups 17, part_check 6, part_segments 6).
+// Node ids: A(r) = 2 r for r in [0, n] (A(n) is the end), B(r) = 2 r + 1.
 //
 // A short-row scan adds at least C_store per row, so it is bounded by
 // capacity / C_store; costs without that bound (C_store <= 0, a negative
@@ -29,12 +41,9 @@
 // CWLB_UNSUPPORTED here and stay with the host partition.
 #pragma clang fp contract(off)
 
-#include <rocprim/device/device_scan.hpp>
-
 #include <algorithm>
 #include <climits>
 #include <cmath>
-#include <vector>
 
 #include "internal.h"
 #include "partition_sim.h"
@@ -44,151 +53,401 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr long long kMaxScan = 1 << 16;
+// Rows per block of part_blocks and part_emit.  2 * kRows nodes of 8 bytes
+// (their jump and task count) are 32 KB of LDS: 4 work-groups per CU.
+constexpr int kRows = 2048;
+constexpr int kThreads = 512;
+constexpr int kPer = 2 * kRows / kThreads;  // nodes per thread
+// Segments of a long row from which a whole wave of a later launch writes
+// them, not a lane, and such rows that a block sets aside (in the LDS of its
+// jumps).
+constexpr int kManySegments = 64;
+constexpr int kMaxMany = 400;
 
 using part::PartParams;
 using part::Emitter;
-using part::simulate;
 using part::full_w;
+using part::simulate_from;
 
-__global__ void __launch_bounds__(kBlock)
-part_flags(PartParams p, int* __restrict__ is_long)
+// What the kernels hand on; one per context, cleared by part_clear.
+struct PartState {
+    int decreasing;  // some offset is smaller than the one before
+    int overrun;     // a row scan exceeded its bound
+    int n_many;      // rows of many segments set aside
+    unsigned long long n_long;
+    long long total;
+};
+
+// A chain node at which a block or group is entered, and the index of the
+// first task emitted from it; node kNone: the chain passes it by.
+struct Entry {
+    unsigned node;
+    long long first;
+};
+constexpr unsigned kNone = 0xffffffffu;
+
+// The node at which the chain leaves a block or group, and the tasks up to
+// there.
+struct BlockExit {
+    unsigned node;
+    unsigned count;
+};
+struct GroupExit {
+    unsigned node;
+    long long count;
+};
+
+struct Layout {
+    int nb;        // blocks of kRows rows
+    int per;       // blocks per group
+    int ng;        // groups
+    int cand;      // rows of a block at which the chain may enter it
+    PartState* state;
+    BlockExit* block_exit;  // nb x cand x {A, B}
+    GroupExit* group_exit;  // ng x cand x {A, B}
+    Entry* block_entry;     // nb
+    Entry* group_entry;     // ng
+};
+
+static_assert(sizeof(PartState) <= 64, "the workspace's first 64 bytes");
+
+__global__ void part_clear(PartState* __restrict__ st)
 {
-    const int r = blockIdx.x * kBlock + threadIdx.x;
-    if (r < p.n) is_long[r] = !(full_w(p, r) <= p.cap) ? 1 : 0;
+    st->decreasing = 0;
+    st->overrun = 0;
+    st->n_many = 0;
+    st->n_long = 0;
+    st->total = 0;
 }
 
+// count: the long rows are counted too (only the largest graphs need them).
 __global__ void __launch_bounds__(kBlock)
-part_compact(int n, const int* __restrict__ is_long, const int* __restrict__ scan,
-             int* __restrict__ long_row, int* __restrict__ long_idx)
+part_check(PartParams p, int count, PartState* __restrict__ st)
 {
-    const int r = blockIdx.x * kBlock + threadIdx.x;
-    if (r >= n) return;
-    if (is_long[r]) {
-        long_row[scan[r]] = r;
-        long_idx[r] = scan[r];
-    } else {
-        long_idx[r] = -1;
+    int mine = 0;
+    bool falls = false;
+    const long long stride = static_cast<long long>(gridDim.x) * kBlock;
+    for (long long r = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x; r < p.n;
+         r += stride) {
+        const int row = static_cast<int>(r);
+        falls |= p.rp[row + 1] < p.rp[row];
+        if (count) mine += !(full_w(p, row) <= p.cap) ? 1 : 0;
+    }
+    if (__ballot(falls) != 0ull && (threadIdx.x & 63) == 0) atomicOr(&st->decreasing, 1);
+    if (count) atomicAdd(&st->n_long, static_cast<unsigned long long>(mine));
+}
+
+// The local index of a node of the block that starts at row b0: the A nodes
+// first, then the B nodes.
+__device__ __forceinline__ int local_of(unsigned node, unsigned b0)
+{
+    return static_cast<int>((node >> 1) - b0) + ((node & 1u) ? kRows : 0);
+}
+
+// Fills jump / cnt with the next node and the task count of every node of
+// the block of rows [b0, b1).  Nodes that no chain visits (B of a short
+// row) jump to the end.
+__device__ __forceinline__ void block_nodes(const PartParams& p, bool search, unsigned b0,
+                                            unsigned b1, unsigned* __restrict__ jump,
+                                            unsigned* __restrict__ cnt, int* __restrict__ overrun)
+{
+#pragma unroll 1
+    for (int k = 0; k < kPer; ++k) {
+        const int x = threadIdx.x + k * kThreads;
+        const bool is_b = x >= kRows;
+        const unsigned row = b0 + (is_b ? x - kRows : x);
+        unsigned to = 2u * static_cast<unsigned>(p.n);
+        unsigned c = 0;
+        if (row < b1) {
+            const int r = static_cast<int>(row);
+            if (!is_b || !(full_w(p, r) <= p.cap)) {
+                Emitter em{nullptr, 0};
+                int over = 0;
+                int next = p.n;
+                bool next_b = false;
+                simulate_from(p, r, is_b, search, em, &over, &next, &next_b);
+                if (over) *overrun = 1;
+                to = 2u * static_cast<unsigned>(next) + (next_b ? 1u : 0u);
+                c = static_cast<unsigned>(em.count);
+            }
+        }
+        jump[x] = to;
+        cnt[x] = c;
     }
 }
 
-__global__ void __launch_bounds__(kBlock)
-part_transitions(PartParams p, long long V, int* __restrict__ next, int* __restrict__ cnt,
-                 int* __restrict__ status)
+// One doubling step: every node whose jump stays in the block takes the
+// jump and the tasks of the node it leads to.  Returns whether any node of
+// the work-group still jumps inside the block.
+__device__ __forceinline__ bool double_step(unsigned b0, unsigned limit,
+                                            unsigned* __restrict__ jump,
+                                            unsigned* __restrict__ cnt)
 {
-    const long long x = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
-    if (x >= V) return;
-    Emitter em{nullptr, 0};
-    int overrun = 0;
-    next[x] = simulate(p, static_cast<int>(x), em, &overrun);
-    cnt[x] = static_cast<int>(em.count);
-    if (overrun) atomicOr(status, 1);
-}
-
-// levels[0] = 1 + the first k with J_k(A(0)) == n (J_k = 2^k steps; the
-// J arrays are consecutive, V entries each), or 0 if none of the L reaches
-// the end.
-__global__ void part_levels(const int* __restrict__ J, long long V, int L, int n,
-                            int* __restrict__ levels)
-{
-    int found = 0;
-    for (int k = 0; k < L; ++k) {
-        if (J[static_cast<long long>(k) * V] == n) {
-            found = k + 1;
-            break;
+    unsigned j[kPer];
+    unsigned c[kPer];
+    bool inside = false;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int x = threadIdx.x + k * kThreads;
+        j[k] = jump[x];
+        c[k] = cnt[x];
+        if (j[k] < limit) {
+            const int y = local_of(j[k], b0);
+            j[k] = jump[y];
+            c[k] += cnt[y];
+            inside |= j[k] < limit;
         }
     }
-    *levels = found;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int x = threadIdx.x + k * kThreads;
+        jump[x] = j[k];
+        cnt[x] = c[k];
+    }
+    return __syncthreads_or(inside) != 0;
+}
+
+__global__ void __launch_bounds__(kThreads)
+part_blocks(PartParams p, Layout l)
+{
+    __shared__ unsigned jump[2 * kRows];
+    __shared__ unsigned cnt[2 * kRows];
+    const unsigned b0 = blockIdx.x * static_cast<unsigned>(kRows);
+    const unsigned b1 = min(b0 + static_cast<unsigned>(kRows), static_cast<unsigned>(p.n));
+    const unsigned limit = 2u * b1;  // nodes from here on are outside
+    const bool search = p.cap >= 0.0 && l.state->decreasing == 0;
+    int over = 0;
+    block_nodes(p, search, b0, b1, jump, cnt, &over);
+    if (over) atomicOr(&l.state->overrun, 1);
+    __syncthreads();
+    while (double_step(b0, limit, jump, cnt)) {
+    }
+    BlockExit* out = l.block_exit + static_cast<size_t>(blockIdx.x) * l.cand * 2;
+    for (int i = threadIdx.x; i < 2 * l.cand; i += kThreads) {
+        const int x = (i >> 1) + ((i & 1) ? kRows : 0);
+        out[i] = BlockExit{jump[x], cnt[x]};
+    }
+    if (threadIdx.x == 0) l.block_entry[blockIdx.x] = Entry{kNone, 0};
+}
+
+// The place of a node in the exits of its block (its row is one of the
+// block's first cand: a chain enters no block elsewhere; a node that would,
+// in a chain that an overrun cut short, is treated as the end).
+__device__ __forceinline__ bool exit_index(const Layout& l, unsigned node, unsigned end, int* block,
+                                           int* i)
+{
+    if (node >= end) return false;
+    const unsigned row = node >> 1;
+    *block = static_cast<int>(row / kRows);
+    const int at = static_cast<int>(row % kRows);
+    *i = 2 * at + static_cast<int>(node & 1u);
+    return at < l.cand;
 }
 
 __global__ void __launch_bounds__(kBlock)
-part_double(long long V, const int* __restrict__ src, int* __restrict__ dst)
+part_groups(int n, Layout l)
 {
-    const long long x = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
-    if (x < V) dst[x] = src[src[x]];
+    const long long t = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
+    const long long all = static_cast<long long>(l.ng) * l.cand * 2;
+    if (t >= all) return;
+    const int g = static_cast<int>(t / (2 * l.cand));
+    const int i0 = static_cast<int>(t % (2 * l.cand));
+    const unsigned end = 2u * static_cast<unsigned>(n);
+    const int last = min((g + 1) * l.per, l.nb);  // first block past the group
+    int block = g * l.per;
+    int i = i0;
+    unsigned node = 2u * (static_cast<unsigned>(block) * kRows + static_cast<unsigned>(i0 >> 1)) +
+                    static_cast<unsigned>(i0 & 1);
+    long long count = 0;
+    while (exit_index(l, node, end, &block, &i) && block < last) {
+        const BlockExit e = l.block_exit[static_cast<size_t>(block) * l.cand * 2 + i];
+        node = e.node;
+        count += e.count;
+    }
+    l.group_exit[t] = GroupExit{node, count};
+    if (i0 == 0) l.group_entry[g] = Entry{kNone, 0};
 }
 
-// Round of the chain expansion: positions pos = i * 2 * half get their
-// successor at pos + half from jump table J (2^j steps, half = 2^j).
-__global__ void __launch_bounds__(kBlock)
-part_expand(long long count, long long half, const int* __restrict__ J, int* __restrict__ chain)
+__global__ void __launch_bounds__(1024)
+part_walk(int n, Layout l)
 {
-    const long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
-    if (i >= count) return;
-    const long long pos = i * 2 * half;
-    chain[pos + half] = J[chain[pos]];
-}
-
-__global__ void __launch_bounds__(kBlock)
-part_chain_counts(long long len, int end, const int* __restrict__ chain,
-                  const int* __restrict__ cnt, long long* __restrict__ c)
-{
-    const long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
-    if (i < len) c[i] = chain[i] == end ? 0 : cnt[chain[i]];
-}
-
-__global__ void __launch_bounds__(kBlock)
-part_emit(PartParams p, long long len, const int* __restrict__ chain,
-          const long long* __restrict__ offsets, cwlb_task* __restrict__ out)
-{
-    const long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
-    if (i >= len || chain[i] == p.n) return;
-    Emitter em{out + offsets[i], 0};
-    int overrun = 0;
-    (void)simulate(p, chain[i], em, &overrun);
-}
-
-// Owning device allocation; movable, not copyable (the jump tables live in
-// a growing vector).
-struct Mem {
-    void* p = nullptr;
-    Mem() = default;
-    Mem(const Mem&) = delete;
-    Mem& operator=(const Mem&) = delete;
-    Mem(Mem&& o) noexcept : p(o.p) { o.p = nullptr; }
-    Mem& operator=(Mem&& o) noexcept
-    {
-        if (this != &o) {
-            if (p) (void)hipFree(p);
-            p = o.p;
-            o.p = nullptr;
+    const unsigned end = 2u * static_cast<unsigned>(n);
+    if (threadIdx.x == 0) {
+        unsigned node = 0;
+        long long at = 0;
+        int block = 0, i = 0;
+        while (exit_index(l, node, end, &block, &i)) {
+            const int g = block / l.per;
+            // A group is entered at its first block, or (a task longer than
+            // a block) at a later one; then its blocks lead out of it.
+            l.group_entry[g] = Entry{node, at};
+            if (block == g * l.per) {
+                const GroupExit e = l.group_exit[static_cast<size_t>(g) * l.cand * 2 + i];
+                node = e.node;
+                at += e.count;
+            } else {
+                const int last = min((g + 1) * l.per, l.nb);
+                while (exit_index(l, node, end, &block, &i) && block < last) {
+                    const BlockExit e = l.block_exit[static_cast<size_t>(block) * l.cand * 2 + i];
+                    node = e.node;
+                    at += e.count;
+                }
+            }
         }
-        return *this;
+        l.state->total = at;
     }
-    ~Mem()
-    {
-        if (p) (void)hipFree(p);
+    __syncthreads();
+    for (int g = threadIdx.x; g < l.ng; g += 1024) {
+        Entry e = l.group_entry[g];
+        if (e.node == kNone) continue;
+        const int last = min((g + 1) * l.per, l.nb);
+        int block = 0, i = 0;
+        while (exit_index(l, e.node, end, &block, &i) && block < last) {
+            l.block_entry[block] = e;
+            const BlockExit x = l.block_exit[static_cast<size_t>(block) * l.cand * 2 + i];
+            e.node = x.node;
+            e.first += x.count;
+        }
     }
-    hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 1); }
-    template <class T>
-    T* as() const
+}
+
+// Writes a node's tasks; the segments of a row with many of them are set
+// aside while there is room.
+struct ManySegments {
+    int g, L, off, k;
+    unsigned at;  // their first task, from the block's on
+};
+struct SetAside {
+    ManySegments row;
+    int pad;
+    long long first;  // the block's first task
+};
+// Kept in the LDS of the jumps, with the list of the chain's nodes.
+static_assert(sizeof(ManySegments) * kMaxMany + sizeof(unsigned short) * 2 * kRows <=
+                  sizeof(unsigned) * 2 * kRows,
+              "the jumps' LDS");
+struct LaneEmitter {
+    cwlb_task* out;
+    unsigned count;
+    ManySegments* many;
+    int* n_many;
+    __device__ void emit(int s, int e, int fo, int last)
     {
-        return static_cast<T*>(p);
+        if (s < e) out[count++] = cwlb_task{s, e, fo, last};
+    }
+    __device__ void segments(int g, int L, int off, int S, int k)
+    {
+        if (k >= kManySegments) {
+            const int i = atomicAdd(n_many, 1);
+            if (i < kMaxMany) {
+                many[i] = ManySegments{g, L, off, k, count};
+                count += static_cast<unsigned>(k);
+                return;
+            }
+        }
+        for (int i = 0; i < k; ++i, off += S)
+            out[count++] = cwlb_task{i == 0 ? g : L, L + 1, off, off + S};
     }
 };
 
-template <class In, class Out>
-cwlb_status exclusive_scan(hipStream_t st, In in, Out out, size_t n)
+__global__ void __launch_bounds__(kThreads)
+part_emit(PartParams p, Layout l, SetAside* __restrict__ aside, cwlb_task* __restrict__ out,
+          long long capacity)
 {
-    using T = typename std::iterator_traits<Out>::value_type;
-    size_t bytes = 0;
-    CWLB_HIP_TRY(rocprim::exclusive_scan(nullptr, bytes, in, out, T(0), n, rocprim::plus<T>(), st));
-    Mem temp;
-    CWLB_HIP_TRY(temp.alloc(bytes));
-    CWLB_HIP_TRY(rocprim::exclusive_scan(temp.p, bytes, in, out, T(0), n, rocprim::plus<T>(), st));
-    CWLB_HIP_TRY(hipStreamSynchronize(st));
-    return CWLB_OK;
+    __shared__ unsigned jump[2 * kRows];
+    __shared__ unsigned cnt[2 * kRows];
+    __shared__ unsigned char on_chain[2 * kRows];
+    __shared__ int n_many;
+    __shared__ int n_nodes;
+    __shared__ int aside_at;
+    const Entry entry = l.block_entry[blockIdx.x];
+    if (entry.node == kNone || l.state->total > capacity || l.state->overrun) return;
+    const unsigned b0 = blockIdx.x * static_cast<unsigned>(kRows);
+    const unsigned b1 = min(b0 + static_cast<unsigned>(kRows), static_cast<unsigned>(p.n));
+    const unsigned limit = 2u * b1;
+    const bool search = p.cap >= 0.0 && l.state->decreasing == 0;
+    const int first = local_of(entry.node, b0);
+    int over = 0;
+    block_nodes(p, search, b0, b1, jump, cnt, &over);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int x = threadIdx.x + k * kThreads;
+        on_chain[x] = x == first;
+    }
+    if (threadIdx.x == 0) n_many = n_nodes = 0;
+    __syncthreads();
+    // After k rounds the marks hold the first 2^k nodes of the chain (and
+    // nothing but nodes of it): every marked node marks the node its jump
+    // of 2^k steps leads to, then the jumps double.
+    for (bool more = true; more;) {
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int x = threadIdx.x + k * kThreads;
+            if (on_chain[x] && jump[x] < limit) on_chain[local_of(jump[x], b0)] = 1;
+        }
+        __syncthreads();
+        more = double_step(b0, limit, jump, cnt);
+    }
+    // cnt[x] is now the number of tasks from node x to the block's exit; the
+    // jumps are done with, and their place takes the chain's nodes, listed so
+    // that no lane idles on a node off the chain, and the rows set aside.
+    cwlb_task* const mine = out + entry.first;
+    const unsigned from_entry = cnt[first];
+    auto* const nodes = reinterpret_cast<unsigned short*>(jump);
+    ManySegments* const many = reinterpret_cast<ManySegments*>(nodes + 2 * kRows);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int x = threadIdx.x + k * kThreads;
+        const unsigned long long m = __ballot(on_chain[x]);
+        int at = 0;
+        if ((threadIdx.x & 63) == 0 && m) at = atomicAdd(&n_nodes, static_cast<int>(__popcll(m)));
+        at = __shfl(at, 0);
+        if (on_chain[x])
+            nodes[at + __popcll(m & ((1ull << (threadIdx.x & 63)) - 1ull))] =
+                static_cast<unsigned short>(x);
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int k = threadIdx.x; k < n_nodes; k += kThreads) {
+        const int x = nodes[k];
+        const bool is_b = x >= kRows;
+        LaneEmitter em{mine, from_entry - cnt[x], many, &n_many};
+        int next = 0;
+        bool next_b = false;
+        simulate_from(p, static_cast<int>(b0) + (is_b ? x - kRows : x), is_b, search, em, &over,
+                      &next, &next_b);
+    }
+    __syncthreads();
+    const int nm = min(n_many, kMaxMany);
+    if (nm == 0) return;
+    if (threadIdx.x == 0) aside_at = atomicAdd(&l.state->n_many, nm);
+    __syncthreads();
+    for (int i = threadIdx.x; i < nm; i += kThreads)
+        aside[aside_at + i] = SetAside{many[i], 0, entry.first};
+}
+
+// The rows set aside, a wave each: the hub rows are neighbours in the order,
+// and one work-group alone writes 16-byte tasks no faster than 30 GB/s (the
+// R-MAT graph's last block: 160 us).
+__global__ void __launch_bounds__(kBlock)
+part_segments(int S, const PartState* __restrict__ st, const SetAside* __restrict__ aside,
+              cwlb_task* __restrict__ out)
+{
+    const int n = st->n_many;
+    const int waves = gridDim.x * (kBlock / 64);
+    for (int i = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); i < n; i += waves) {
+        const SetAside a = aside[i];
+        const ManySegments d = a.row;
+        cwlb_task* const to = out + a.first + d.at;
+        for (int j = threadIdx.x & 63; j < d.k; j += 64) {
+            const int off = d.off + j * S;
+            to[j] = cwlb_task{j == 0 ? d.g : d.L, d.L + 1, off, off + S};
+        }
+    }
 }
 
 unsigned grid_for(long long n) { return static_cast<unsigned>((n + kBlock - 1) / kBlock); }
-
-// Clears one or two words with a kernel rather than hipMemsetAsync (memset
-// nodes are kept out of anything a caller may record into a graph).
-template <class T>
-__global__ void part_clear(T* __restrict__ a, T* __restrict__ b)
-{
-    *a = T(0);
-    if (b) *b = T(0);
-}
 
 }  // namespace
 
@@ -224,103 +483,77 @@ cwlb_status launch_partition(cwlb_ctx* ctx, const int32_t* rp, int32_t n,
     p.max_scan = static_cast<long long>(cap / p.cs * (1.0 + 1e-6)) + 4;
 
     (void)hipGetLastError();  // a stale error of an earlier call must not be reported here
-    // Long rows and their compact indices.
-    Mem is_long, scan, long_row, long_idx, status;
-    CWLB_HIP_TRY(is_long.alloc(sizeof(int) * (n + 1)));
-    CWLB_HIP_TRY(scan.alloc(sizeof(int) * (n + 1)));
-    CWLB_HIP_TRY(long_idx.alloc(sizeof(int) * n));
-    CWLB_HIP_TRY(status.alloc(sizeof(int)));
-    hipLaunchKernelGGL(part_clear<int>, dim3(1), dim3(1), 0, st, status.as<int>(),
-                       is_long.as<int>() + n);
-    CWLB_LAUNCH_CHECK("part_clear");
-    hipLaunchKernelGGL(part_flags, dim3(grid_for(n)), dim3(kBlock), 0, st, p, is_long.as<int>());
-    CWLB_LAUNCH_CHECK("part_flags");
-    cwlb_status s = exclusive_scan(st, is_long.as<int>(), scan.as<int>(), static_cast<size_t>(n) + 1);
-    if (s != CWLB_OK) return s;
-    int n_long = 0;
-    CWLB_HIP_TRY(hipMemcpyAsync(&n_long, scan.as<int>() + n, sizeof(int), hipMemcpyDeviceToHost, st));
-    CWLB_HIP_TRY(hipStreamSynchronize(st));
-    CWLB_HIP_TRY(long_row.alloc(sizeof(int) * std::max(n_long, 1)));
-    hipLaunchKernelGGL(part_compact, dim3(grid_for(n)), dim3(kBlock), 0, st, n, is_long.as<int>(),
-                       scan.as<int>(), long_row.as<int>(), long_idx.as<int>());
-    CWLB_LAUNCH_CHECK("part_compact");
-    p.long_row = long_row.as<int>();
-    p.long_idx = long_idx.as<int>();
+    Layout l{};
+    l.nb = (n - 1) / kRows + 1;
+    l.per = 1;
+    while (static_cast<long long>(l.per) * l.per < l.nb) ++l.per;
+    l.ng = (l.nb - 1) / l.per + 1;
+    // A task that starts before the block ends at most max_scan rows on, and
+    // the long row it then takes is one more.
+    l.cand = static_cast<int>(std::min<long long>(kRows, std::max<long long>(p.max_scan, 0) + 2));
+    const size_t exits = static_cast<size_t>(l.cand) * 2;
+    const size_t b_state = 64;
+    const size_t b_group_exit = sizeof(GroupExit) * exits * l.ng;
+    const size_t b_block_exit = sizeof(BlockExit) * exits * l.nb;
+    const size_t b_block_entry = sizeof(Entry) * l.nb;
+    const size_t b_group_entry = sizeof(Entry) * l.ng;
+    // Every row set aside has at least kManySegments tasks of its own, and
+    // none is when the tasks exceed the capacity.
+    const bool emit = out && capacity_tasks > 0;
+    const size_t b_aside =
+        emit ? sizeof(SetAside) * std::min<long long>(capacity_tasks / kManySegments, n) : 0;
+    const size_t want = b_state + b_group_exit + b_block_exit + b_block_entry + b_group_entry +
+                        b_aside;
+    if (want > ctx->part_bytes) {
+        if (ctx->d_part) CWLB_HIP_TRY(hipFree(ctx->d_part));
+        ctx->d_part = nullptr;
+        ctx->part_bytes = 0;
+        CWLB_HIP_TRY(hipMalloc(&ctx->d_part, want));
+        ctx->part_bytes = want;
+    }
+    char* at = static_cast<char*>(ctx->d_part);
+    l.state = reinterpret_cast<PartState*>(at);
+    at += b_state;
+    l.group_exit = reinterpret_cast<GroupExit*>(at);
+    at += b_group_exit;
+    l.block_entry = reinterpret_cast<Entry*>(at);
+    at += b_block_entry;
+    l.group_entry = reinterpret_cast<Entry*>(at);
+    at += b_group_entry;
+    auto* const aside = reinterpret_cast<SetAside*>(at);
+    at += b_aside;
+    l.block_exit = reinterpret_cast<BlockExit*>(at);
 
-    // 1. transitions of every node.
-    const long long V = static_cast<long long>(n) + 1 + n_long;
-    if (V > INT_MAX) return fail(CWLB_UNSUPPORTED, "cwlb_partition_device: too many rows");
-    // The chain from A(0) has at most V fresh nodes, so L doubling levels
-    // (2^(L-1) >= V) always reach the end; all are computed back to back
-    // in one allocation, then one read-back finds how many were needed.
-    int L = 1;
-    while ((1LL << (L - 1)) < V) ++L;
-    Mem cnt, Jall;
-    CWLB_HIP_TRY(cnt.alloc(sizeof(int) * V));
-    CWLB_HIP_TRY(Jall.alloc(sizeof(int) * static_cast<size_t>(V) * L + sizeof(int)));
-    int* const J0 = Jall.as<int>();
-    auto J = [&](int k) { return J0 + static_cast<long long>(k) * V; };
-    int* const d_levels = J0 + static_cast<long long>(L) * V;
-    hipLaunchKernelGGL(part_transitions, dim3(grid_for(V)), dim3(kBlock), 0, st, p, V,
-                       J(0), cnt.as<int>(), status.as<int>());
-    CWLB_LAUNCH_CHECK("part_transitions");
-    // 2. doubling: J_{k+1} = J_k o J_k.
-    for (int k = 1; k < L; ++k) {
-        hipLaunchKernelGGL(part_double, dim3(grid_for(V)), dim3(kBlock), 0, st, V, J(k - 1), J(k));
-        CWLB_LAUNCH_CHECK("part_double");
-    }
-    hipLaunchKernelGGL(part_levels, dim3(1), dim3(1), 0, st, J0, V, L, n, d_levels);
-    CWLB_LAUNCH_CHECK("part_levels");
-    int host_status[2] = {0, 0};
-    CWLB_HIP_TRY(hipMemcpyAsync(&host_status[0], status.p, sizeof(int), hipMemcpyDeviceToHost, st));
-    CWLB_HIP_TRY(hipMemcpyAsync(&host_status[1], d_levels, sizeof(int), hipMemcpyDeviceToHost, st));
-    CWLB_HIP_TRY(hipStreamSynchronize(st));
-    if (host_status[0]) return fail(CWLB_RUNTIME_ERROR, "cwlb_partition_device: a row scan exceeded its bound");
-    const int levels = host_status[1];
-    if (levels <= 0) return fail(CWLB_RUNTIME_ERROR, "cwlb_partition_device: chain too long");
-    // J[levels-1] maps A(0) to the end: the chain has at most 2^(levels-1)
-    // fresh nodes before the end.
-    const long long len = 1LL << (levels - 1);
-    Mem chain, counts, offsets;
-    CWLB_HIP_TRY(chain.alloc(sizeof(int) * len));
-    hipLaunchKernelGGL(part_clear<int>, dim3(1), dim3(1), 0, st, chain.as<int>(),
-                       static_cast<int*>(nullptr));
+    (void)hipGetLastError();  // a stale error of an earlier call must not be reported here
+    hipLaunchKernelGGL(part_clear, dim3(1), dim3(1), 0, st, l.state);
     CWLB_LAUNCH_CHECK("part_clear");
-    // 3. expansion: positions that are multiples of 2 * half get their
-    // successor half steps on.
-    for (int j = levels - 2; j >= 0; --j) {
-        const long long half = 1LL << j;
-        const long long count = len / (2 * half);
-        hipLaunchKernelGGL(part_expand, dim3(grid_for(count)), dim3(kBlock), 0, st, count, half,
-                           J(j), chain.as<int>());
-        CWLB_LAUNCH_CHECK("part_expand");
-    }
-    // 4. task offsets of the chain nodes.
-    CWLB_HIP_TRY(counts.alloc(sizeof(long long) * (len + 1)));
-    CWLB_HIP_TRY(offsets.alloc(sizeof(long long) * (len + 1)));
-    hipLaunchKernelGGL(part_clear<long long>, dim3(1), dim3(1), 0, st,
-                       counts.as<long long>() + len, static_cast<long long*>(nullptr));
-    CWLB_LAUNCH_CHECK("part_clear");
-    hipLaunchKernelGGL(part_chain_counts, dim3(grid_for(len)), dim3(kBlock), 0, st, len, n,
-                       chain.as<int>(), cnt.as<int>(), counts.as<long long>());
-    CWLB_LAUNCH_CHECK("part_chain_counts");
-    s = exclusive_scan(st, counts.as<long long>(), offsets.as<long long>(),
-                       static_cast<size_t>(len) + 1);
-    if (s != CWLB_OK) return s;
-    long long total = 0;
-    CWLB_HIP_TRY(hipMemcpyAsync(&total, offsets.as<long long>() + len, sizeof(long long),
-                                hipMemcpyDeviceToHost, st));
-    CWLB_HIP_TRY(hipStreamSynchronize(st));
-    *n_tasks = total;
-    if (total > capacity_tasks || (!out && total > 0))
-        return fail(CWLB_INSUFFICIENT, "cwlb_partition_device: output buffer too small");
-    // 5. the tasks.
-    if (total > 0) {
-        hipLaunchKernelGGL(part_emit, dim3(grid_for(len)), dim3(kBlock), 0, st, p, len,
-                           chain.as<int>(), offsets.as<long long>(), out);
+    hipLaunchKernelGGL(part_check, dim3(std::min(grid_for(n), 4096u)), dim3(kBlock), 0, st, p,
+                       n >= INT_MAX / 2 ? 1 : 0, l.state);
+    CWLB_LAUNCH_CHECK("part_check");
+    hipLaunchKernelGGL(part_blocks, dim3(l.nb), dim3(kThreads), 0, st, p, l);
+    CWLB_LAUNCH_CHECK("part_blocks");
+    hipLaunchKernelGGL(part_groups, dim3(grid_for(static_cast<long long>(exits) * l.ng)),
+                       dim3(kBlock), 0, st, n, l);
+    CWLB_LAUNCH_CHECK("part_groups");
+    hipLaunchKernelGGL(part_walk, dim3(1), dim3(1024), 0, st, n, l);
+    CWLB_LAUNCH_CHECK("part_walk");
+    if (emit) {
+        hipLaunchKernelGGL(part_emit, dim3(l.nb), dim3(kThreads), 0, st, p, l, aside, out,
+                           static_cast<long long>(capacity_tasks));
         CWLB_LAUNCH_CHECK("part_emit");
+        hipLaunchKernelGGL(part_segments, dim3(1024), dim3(kBlock), 0, st, p.S, l.state, aside, out);
+        CWLB_LAUNCH_CHECK("part_segments");
     }
+    PartState state{};
+    CWLB_HIP_TRY(hipMemcpyAsync(&state, l.state, sizeof state, hipMemcpyDeviceToHost, st));
     CWLB_HIP_TRY(hipStreamSynchronize(st));
+    if (static_cast<long long>(n) + 1 + static_cast<long long>(state.n_long) > INT_MAX)
+        return fail(CWLB_UNSUPPORTED, "cwlb_partition_device: too many rows");
+    if (state.overrun)
+        return fail(CWLB_RUNTIME_ERROR, "cwlb_partition_device: a row scan exceeded its bound");
+    *n_tasks = state.total;
+    if (state.total > capacity_tasks || (!out && state.total > 0))
+        return fail(CWLB_INSUFFICIENT, "cwlb_partition_device: output buffer too small");
     return CWLB_OK;
 }
 

@@ -52,98 +52,187 @@ struct Emitter {
             ++count;
         }
     }
+    // k segments of S nonzeros of row L from nonzero off on; the first
+    // task starts at row g.
+    CWLB_HD void segments(int g, int L, int off, int S, int k)
+    {
+        if (out) {
+            for (int i = 0; i < k; ++i, off += S)
+                out[count + i] = cwlb_task{i == 0 ? g : L, L + 1, off, off + S};
+        }
+        count += k;
+    }
 };
 
-// Simulates the host state machine from fresh node x to the next fresh
-// node (returned), emitting the tasks closed on the way.  *overrun is set
-// when a short-row scan exceeds its bound (the caller then fails the call).
-CWLB_HD inline int simulate(const PartParams& p, int x, Emitter& em, int* overrun)
+// Where a pack of whole rows from row x on stops: at row n, at a long row
+// (full weight above the capacity) or at a row that no longer fits.  acc is
+// the packed load, `exact` whether it is the host's sum to the last bit.
+struct Pack {
+    int row;
+    bool is_long;
+    bool exact;
+    double acc;
+};
+
+// The host's loop: one rounded addition per row, in its order.  False when
+// the scan exceeds its bound.
+CWLB_HD inline bool pack_scan(const PartParams& p, int x, Pack& k)
+{
+    k.row = x;
+    k.is_long = false;
+    k.exact = true;
+    k.acc = 0.0;
+    long long steps = 0;
+    while (k.row < p.n) {
+        if (++steps > p.max_scan) return false;
+        const double wr = full_w(p, k.row);
+        if (!(wr <= p.cap)) {
+            k.is_long = true;
+            return true;
+        }
+        if (!(k.acc == 0.0 || k.acc + wr <= p.cap)) return true;
+        k.acc += wr;
+        ++k.row;
+    }
+    return true;
+}
+
+// The same stop by binary search, for offsets that never decrease and a
+// capacity >= 0.  In real arithmetic the load of rows [x, r) is
+//     F(r) = (C_compute + C_load) * (rp[r] - rp[x]) + C_store * (r - x),
+// which grows with r, and a row is accepted exactly while the load with it
+// stays within the capacity (a long row never does).  The host's sum of k
+// rows rounds 2k + k - 1 times, each by at most 2^-53 of a load that is at
+// most the capacity, and F as computed here three times: they differ by
+// less than margin = capacity * (max_scan + 16) * 2^-52 while k <= max_scan
+// (a row's weight rounds twice, its error relative to the row: together at
+// most 2^-52 of the load; the k - 1 additions at most (k - 1) * 2^-53).  A
+// stop whose two neighbouring loads are further than that from the capacity
+// is therefore the host's; any other is left to pack_scan.
+CWLB_HD inline bool pack_search(const PartParams& p, int x, Pack& k)
+{
+    const double margin = p.cap * (static_cast<double>(p.max_scan) + 16.0) * 0x1.0p-52;
+    const int base = p.rp[x];
+    int lo = x;  // the load of [x, lo) is within the capacity
+    int hi = p.n - x > p.max_scan ? x + static_cast<int>(p.max_scan) : p.n;
+    const int end = hi;
+    double f_lo = 0.0;
+    double f_hi = p.wcl * static_cast<double>(p.rp[hi] - base) + p.cs * static_cast<double>(hi - x);
+    if (f_hi <= p.cap) {
+        lo = hi;
+        f_lo = f_hi;
+    }
+    while (hi - lo > 1) {
+        const int mid = lo + (hi - lo) / 2;
+        const double f =
+            p.wcl * static_cast<double>(p.rp[mid] - base) + p.cs * static_cast<double>(mid - x);
+        if (f <= p.cap) {
+            lo = mid;
+            f_lo = f;
+        } else {
+            hi = mid;
+            f_hi = f;
+        }
+    }
+    if ((lo > x && !(f_lo <= p.cap - margin)) ||
+        (lo < p.n && (lo == end || !(f_hi >= p.cap + margin))))
+        return pack_scan(p, x, k);
+    k.row = lo;
+    k.is_long = lo < p.n && !(full_w(p, lo) <= p.cap);
+    k.exact = lo == x;
+    k.acc = f_lo;
+    return true;
+}
+
+// Whether a chunk of weight w fits beside the packed load of rows
+// [x, k.row): the host's comparison, decided from F where it lies further
+// than the rounding bound from the capacity, else with the host's sum.
+CWLB_HD inline bool chunk_fits(const PartParams& p, int x, const Pack& k, double w)
+{
+    double acc = k.acc;
+    if (!k.exact) {
+        const double room = p.cap - acc;
+        const double margin = p.cap * (static_cast<double>(p.max_scan) + 32.0) * 0x1.0p-52;
+        if (w <= room - margin) return true;
+        if (w >= room + margin) return false;
+        acc = 0.0;
+        for (int r = x; r < k.row; ++r) acc += full_w(p, r);
+    }
+    return w <= p.cap - acc;
+}
+
+// Simulates the host state machine from the fresh node A(r0) (is_b false)
+// or B(r0) (is_b true) to the next fresh node, (*next_row, *next_b),
+// emitting the tasks closed on the way.  search: the offsets never decrease
+// and the capacity is >= 0, so that packs may be found by search.  *overrun
+// is set when a short-row scan exceeds its bound (the caller then fails the
+// call).
+template <class Em>
+CWLB_HD inline void simulate_from(const PartParams& p, int r0, bool is_b, bool search, Em& em,
+                                  int* overrun, int* next_row, bool* next_b)
 {
     const int n = p.n;
     const int S = p.S;
-    int L, g, fo, off, remaining;
+    int L, g, off, remaining;
     double acc = 0.0;
-    if (x <= n) {
-        // ---- A(x): pack whole rows.
-        if (x == n) return n;
-        int row = x;
-        g = x;
-        fo = 0;
-        long long steps = 0;
-        for (;;) {
-            if (row == n) {
-                if (acc > 0.0 || g < n) em.emit(g, n, fo, 0);
-                return n;
-            }
-            if (++steps > p.max_scan) {
-                *overrun = 1;
-                return n;
-            }
-            const double wr = full_w(p, row);
-            if (!(wr <= p.cap)) break;  // long row
-            if (acc == 0.0 || acc + wr <= p.cap) {
-                acc += wr;
-                ++row;
-                continue;
-            }
-            em.emit(g, row, fo, 0);
-            return row;
+    *next_b = false;
+    if (!is_b) {
+        // ---- A(r0): pack whole rows.
+        *next_row = n;
+        if (r0 == n) return;
+        Pack k;
+        if (!(search ? pack_search(p, r0, k) : pack_scan(p, r0, k))) {
+            *overrun = 1;
+            return;
         }
-        L = row;
+        if (k.row == n) {
+            em.emit(r0, n, 0, 0);
+            return;
+        }
+        if (!k.is_long) {
+            em.emit(r0, k.row, 0, 0);
+            *next_row = k.row;
+            return;
+        }
+        L = k.row;
+        g = L;
         const int deg = degree(p, L);
         off = 0;
         remaining = deg;
-        if (remaining <= 0) return L + 1;  // the host drops the open task here
+        *next_row = L + 1;
+        if (remaining <= 0) return;  // the host drops the open task here
         // Ride the deg % S prefix at the end of the open task.
-        if (!(acc <= 0.0)) {
+        if (!(k.acc <= 0.0)) {
             const int r = deg % S;
-            if (r == 0 || r >= deg) {
-                em.emit(g, L, fo, 0);
-                g = L;
-                fo = 0;
-                acc = 0.0;
-            } else if (chunk_w(p, r) <= p.cap - acc) {
-                em.emit(g, L + 1, fo, r);
-                g = L;
-                fo = r;
-                acc = 0.0;
+            if (r != 0 && r < deg && chunk_fits(p, r0, k, chunk_w(p, r))) {
+                em.emit(r0, L + 1, 0, r);
                 remaining -= r;
-                off += r;
+                off = r;
             } else {
-                em.emit(g, L, fo, 0);
-                g = L;
-                fo = 0;
-                acc = 0.0;
+                em.emit(r0, L, 0, 0);
             }
+        } else {
+            g = r0;
+            acc = k.acc;
         }
     } else {
         // ---- B(L): the prefix of L already belongs to the previous task.
-        L = p.long_row[x - n - 1];
-        const int deg = degree(p, L);
+        L = r0;
         g = L;
-        fo = deg % S;
-        off = fo;
+        const int deg = degree(p, L);
+        off = deg % S;
         remaining = deg - off;
-        if (remaining <= 0) return L + 1;
+        *next_row = L + 1;
+        if (remaining <= 0) return;
     }
     // ---- Segments of at most S nonzeros: every segment but the last closes
     // a task; the last one's load decides the next-prefix absorption.
     const int nseg = (remaining - 1) / S + 1;
     const int last = remaining - (nseg - 1) * S;
     if (nseg > 1) {
-        if (em.out) {
-            for (int i = 0; i < nseg - 1; ++i) {
-                off += S;
-                em.emit(g, L + 1, fo, off);
-                g = L;
-                fo = off;
-            }
-        } else {
-            em.count += nseg - 1;
-            off += (nseg - 1) * S;
-            g = L;
-            fo = off;
-        }
+        em.segments(g, L, off, S, nseg - 1);
+        g = L;
+        off += (nseg - 1) * S;
         acc = 0.0;
     }
     acc += chunk_w(p, last);
@@ -154,13 +243,25 @@ CWLB_HD inline int simulate(const PartParams& p, int x, Emitter& em, int* overru
             const int nd = degree(p, nr);
             const int r2 = nd % S;
             if (r2 != 0 && r2 < nd && !(chunk_w(p, r2) > p.cap - acc)) {
-                em.emit(g, nr + 1, fo, r2);
-                return n + 1 + p.long_idx[nr];
+                em.emit(g, nr + 1, off, r2);
+                *next_row = nr;
+                *next_b = true;
+                return;
             }
         }
     }
-    em.emit(g, L + 1, fo, 0);
-    return L + 1;
+    em.emit(g, L + 1, off, 0);
+}
+
+// The same with compact node ids, A(r) = r and B(r) = n + 1 + long_idx[r],
+// and the host's scan throughout.
+CWLB_HD inline int simulate(const PartParams& p, int x, Emitter& em, int* overrun)
+{
+    const bool is_b = x > p.n;
+    int row = p.n;
+    bool b = false;
+    simulate_from(p, is_b ? p.long_row[x - p.n - 1] : x, is_b, false, em, overrun, &row, &b);
+    return b ? p.n + 1 + p.long_idx[row] : row;
 }
 
 }  // namespace part

@@ -1,0 +1,126 @@
+"""The GPU partition's packing by binary search against the host's loop.
+
+csrc/partition_sim.h finds where a pack of short rows stops by a binary
+search over the row offsets and decides it from one expression where that
+lies further than the rounding bound from the capacity; the host's partition
+adds row by row in double precision.  Compiled for the host, both are run
+from every row of drawn offset arrays under costs with and without exact
+sums (with exact ones loads hit the capacity exactly), and must agree on the
+stop, and so must the next node and the task count of every node.  The GPU
+cases run the blocked partition at the edges of its row blocks against the
+host partition.
+"""
+import ctypes
+import subprocess
+
+import numpy as np
+import pytest
+
+from conftest import PKG, ROOT, SKEWED_COSTS, UNIT_COSTS
+from cwlb_amd import capi
+
+GFX950_COSTS = (0.004519, 0.015617, 0.010667, 0.540499)
+
+SOURCE = r"""
+#include "partition_sim.h"
+using namespace cwlb::part;
+// Rows whose search stops elsewhere than the scan, or whose simulation ends
+// at another node or count; *scans: rows that the search left to the scan.
+extern "C" long long compare(const int* rp, int n, double wcl, double cs, double ca, double cap,
+                             int S, long long max_scan)
+{
+    PartParams p{};
+    p.rp = rp; p.n = n; p.S = S; p.wcl = wcl; p.cs = cs; p.ca = ca; p.cap = cap;
+    p.max_scan = max_scan;
+    long long bad = 0;
+    for (int r = 0; r < n; ++r) {
+        Pack a, b;
+        if (!pack_scan(p, r, a) || !pack_search(p, r, b)) return -1;
+        bad += a.row != b.row || a.is_long != b.is_long;
+        for (int k = 1; k < S; k += 1 + S / 40)
+            bad += chunk_fits(p, r, b, chunk_w(p, k)) != (chunk_w(p, k) <= p.cap - a.acc);
+        for (int is_b = 0; is_b < 2; ++is_b) {
+            if (is_b && full_w(p, r) <= p.cap) continue;
+            int row[2], over = 0;
+            bool nb[2];
+            long long cnt[2];
+            for (int s = 0; s < 2; ++s) {
+                Emitter em{nullptr, 0};
+                simulate_from(p, r, is_b, s, em, &over, &row[s], &nb[s]);
+                cnt[s] = em.count;
+            }
+            bad += over || row[0] != row[1] || nb[0] != nb[1] || cnt[0] != cnt[1];
+        }
+    }
+    return bad;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def compare(tmp_path_factory):
+    d = tmp_path_factory.mktemp("search")
+    (d / "c.cpp").write_text(SOURCE)
+    subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-shared", "-fPIC",
+                    f"-I{ROOT}/include", f"-I{PKG}/csrc", str(d / "c.cpp"), "-o",
+                    str(d / "c.so")], check=True)
+    f = ctypes.CDLL(str(d / "c.so")).compare
+    f.restype = ctypes.c_longlong
+    f.argtypes = [ctypes.c_void_p, ctypes.c_int] + [ctypes.c_double] * 4 + [ctypes.c_int,
+                                                                             ctypes.c_longlong]
+    return f
+
+
+def degrees(kind, rng, n):
+    if kind == "zeros":
+        return np.zeros(n, np.int64)
+    if kind == "equal":
+        return np.full(n, int(rng.integers(1, 12)))
+    if kind == "sorted":
+        return np.sort((rng.pareto(1.1, n) * 2).astype(np.int64).clip(0, 5000))
+    d = rng.integers(0, 9, n)
+    return np.where(rng.random(n) < 0.05, rng.integers(0, 4000, n), d)
+
+
+@pytest.mark.parametrize("costs", [UNIT_COSTS, SKEWED_COSTS, GFX950_COSTS,
+                                   (0.1, 0.2, 0.3, 0.7)], ids=str)
+@pytest.mark.parametrize("kind", ["zeros", "equal", "sorted", "mixed"])
+def test_search_equals_scan(compare, kind, costs):
+    rng = np.random.default_rng(sum(kind.encode()))
+    wcl, cs, ca = costs[0] + costs[1], costs[2], costs[3]
+    for S in (1, 2, 7, 60, 333):
+        rp = np.concatenate([[0], np.cumsum(degrees(kind, rng, 3000))]).astype(np.int32)
+        # The capacity of S, and ones that whole rows fill exactly.
+        for cap in (capi.capacity_from_s(S, costs), wcl * S + cs, cs * S, wcl * S + 3 * cs):
+            max_scan = int(cap / cs * (1.0 + 1e-6)) + 4
+            s = max(1, int((cap - ca) // wcl))
+            assert compare(rp.ctypes.data, len(rp) - 1, wcl, cs, ca, cap, s, max_scan) == 0, (S, cap)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 4097, 20000])
+@pytest.mark.parametrize("kind", ["zeros", "equal", "sorted", "mixed", "hubs"])
+def test_blocked_partition(gpu_ctx, kind, n):
+    """Row counts around the blocks of 2,048 rows; packs shorter and (zero
+    rows under a large capacity) longer than a block; hub rows of 63 to 70
+    segments and more, which the whole work-group writes."""
+    import torch
+    rng = np.random.default_rng(n)
+    if kind == "hubs":
+        d = rng.integers(0, 3, n)
+        at = rng.choice(n, min(n, 150), replace=False)
+        d[at] = rng.integers(300, 2500, len(at))
+    else:
+        d = degrees(kind, rng, n)
+    rp = np.concatenate([[0], np.cumsum(d)]).astype(np.int32)
+    for costs in (UNIT_COSTS, GFX950_COSTS):
+        for S in (5, 61, 20000):
+            cap = capi.capacity_from_s(S, costs)
+            want = capi.partition(rp, costs, cap)
+            d_rp = torch.from_numpy(rp).cuda()
+            T = gpu_ctx.partition_device_count(d_rp, n, costs, cap)
+            assert T == len(want), (costs, S)
+            out = torch.full((T + 1, 4), -9, dtype=torch.int32, device="cuda")
+            assert gpu_ctx.partition_device(d_rp, n, costs, cap, out, T) == T
+            got = out.cpu().numpy()
+            assert np.array_equal(got[:T], want) and (got[T] == -9).all(), (costs, S)
