@@ -303,7 +303,7 @@ cwlb_status cwlb_ctx_destroy(cwlb_ctx* ctx)
     if (ctx->switch_ev) (void)hipEventDestroy(ctx->switch_ev);
     if (ctx->d_status) (void)hipFree(ctx->d_status);
     for (void* p : {static_cast<void*>(ctx->d_run_keys), static_cast<void*>(ctx->d_run_keys_sorted),
-                    static_cast<void*>(ctx->d_run_order), ctx->d_sort_temp, ctx->d_part,
+                    static_cast<void*>(ctx->d_run_order), ctx->d_sort_temp, ctx->d_part, ctx->d_reorder,
                     static_cast<void*>(ctx->d_col_counts), static_cast<void*>(ctx->d_count_hist),
                     static_cast<void*>(ctx->d_hints), static_cast<void*>(ctx->d_phase_bounds),
                     static_cast<void*>(ctx->d_band_col), static_cast<void*>(ctx->d_band_val)})

@@ -54,7 +54,10 @@ struct cwlb_ctx {
     int order_M = 0;
     void* d_sort_temp = nullptr;
     size_t sort_temp_bytes = 0;
-    // Grow-only workspace of the GPU partition.
+    // Grow-only workspaces of the GPU reordering (its sort's temporary
+    // storage is d_sort_temp) and of the GPU partition.
+    void* d_reorder = nullptr;
+    size_t reorder_bytes = 0;
     void* d_part = nullptr;
     size_t part_bytes = 0;
     // Set when a launch under graph capture used d_run_order (resp.

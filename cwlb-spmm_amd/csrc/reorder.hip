@@ -9,11 +9,21 @@
 //      degree needs (rocPRIM): equal degrees keep ascending original ids, so
 //      the order is the reference comparator's (degree, id) order;
 //   3. row_ptr_out = 0 followed by the inclusive scan of the sorted degrees;
-//   4. gather_rows / gather_long: each reordered row copies its entries from
-//      the original row: a lane per row of at most 16 entries; the longer
-//      rows (a suffix of the sorted order) as one contiguous output range
-//      cut into equal chunks, so no wave copies a hub row alone.
-// The call synchronises on the context's stream.
+//   4. gather_windows / gather_long: each reordered row copies its entries
+//      from the original row.  Rows of at most kWindowMax entries go 64 to a
+//      wave, the longer rows (a suffix of the sorted order) as one contiguous
+//      output range cut into equal chunks, so no wave copies a hub row alone;
+//      either way the rows' places are read once, a row per lane, and the
+//      entries copied with coalesced stores, each finding its row by a binary
+//      search in LDS.
+// The call synchronises on the context's stream twice: for the checks, and
+// at the end.  Its buffers are the context's.
+// What bounds it is step 4, which reads and writes 8 bytes an entry in rows of
+// a few entries, and the sort's passes over the keys.  4.2M-row R-MAT graph
+// (65M nonzeros, 1.04 GB of entries both ways): 1,282 us per call with a lane
+// per row of at most 16 entries (265 us, uncoalesced), threads that walked
+// the longer rows' offsets (347 us) and buffers allocated by the call; 569 us
+// now, 151 us and 209 us (2.9 TB/s) for the two copies, 150 for the sort.
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 #include <rocprim/iterator/counting_iterator.hpp>
@@ -24,8 +34,12 @@ namespace cwlb {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kLaneRowMax = 16;
+constexpr int kWindowMax = 64;           // entries of a row of gather_windows
 constexpr int kLongChunk = kBlock * 16;  // entries per gather_long block
+// Rows that a chunk of gather_long touches at most: all of more than
+// kWindowMax entries but the first and the last.
+constexpr int kChunkRows = kLongChunk / (kWindowMax + 1) + 2;
+constexpr int kCopy = 4;  // entries per lane in flight
 
 // status bit 0: an offset outside [0, nnz] or a decreasing pair.  Each
 // block writes its maximum degree to block_max[blockIdx.x] (one contended
@@ -60,9 +74,18 @@ degree_keys(const int* __restrict__ rp, int n, long long nnz, unsigned* __restri
     }
 }
 
-// One block: the maximum of the per-block maxima into *out.
+// What the host checks after degree_keys.
+struct ReorderState {
+    int status;
+    unsigned max_deg;
+    int first;  // row_ptr[0]
+    int last;   // row_ptr[n]
+};
+
+// One block: the maximum of the per-block maxima, and row_ptr's ends.
 __global__ void __launch_bounds__(1024)
-reduce_max(const unsigned* __restrict__ v, long long n, unsigned* __restrict__ out)
+reduce_max(const unsigned* __restrict__ v, long long n, const int* __restrict__ rp, int n_rows,
+           ReorderState* __restrict__ out)
 {
     __shared__ unsigned part[1024 / 64];
     unsigned m = 0;
@@ -75,111 +98,176 @@ reduce_max(const unsigned* __restrict__ v, long long n, unsigned* __restrict__ o
     if (threadIdx.x == 0) {
         unsigned r = 0;
         for (int w = 0; w < 1024 / 64; ++w) r = max(r, part[w]);
-        *out = r;
+        out->max_deg = r;
+        out->first = rp[0];
+        out->last = rp[n_rows];
     }
 }
 
-// Rows of at most kLaneRowMax entries: a lane per row.  Longer rows are
-// gathered by gather_long.
-__global__ void __launch_bounds__(kBlock)
-gather_rows(const int* __restrict__ rp, const int* __restrict__ ci, const float* __restrict__ val,
-            const int* __restrict__ origin, const int* __restrict__ rp_out, int n,
-            int* __restrict__ ci_out, float* __restrict__ val_out)
+// The number of leading i in [0, n) for which before(i) holds (true ones
+// first), by one whole wave: 64 probes per round trip.
+template <class Fn>
+__device__ __forceinline__ int wave_partition_point(int n, Fn before)
 {
-    const int r = blockIdx.x * kBlock + threadIdx.x;
-    if (r >= n) return;
-    const int dst = rp_out[r];
-    const int len = rp_out[r + 1] - dst;
-    if (len > kLaneRowMax) return;
-    const int src = rp[origin[r]];
-    for (int j = 0; j < len; ++j) {
-        ci_out[dst + j] = ci[src + j];
-        val_out[dst + j] = val[src + j];
-    }
-}
-
-// long_row[0] = the first reordered row with more than kLaneRowMax entries
-// (n if none): the degrees are sorted ascending, so those rows are a suffix.
-__global__ void find_long_rows(const unsigned* __restrict__ sorted_deg, int n,
-                               int* __restrict__ long_row)
-{
-    int lo = 0, hi = n;
+    int lo = 0, hi = n;  // the point lies in [lo, hi]
     while (lo < hi) {
-        const int mid = lo + (hi - lo) / 2;
-        if (sorted_deg[mid] > static_cast<unsigned>(kLaneRowMax)) hi = mid;
-        else lo = mid + 1;
+        const int step = (hi - lo - 1) / 64 + 1;
+        const long long at = static_cast<long long>(lo) + static_cast<long long>(threadIdx.x & 63) * step;
+        const bool yes = at < hi && before(static_cast<int>(at));
+        const int k = __popcll(__ballot(yes));  // probes lo, lo + step, ... that hold
+        if (k == 0) {
+            hi = lo;
+        } else {
+            const long long next = static_cast<long long>(lo) + static_cast<long long>(k) * step;
+            lo += (k - 1) * step + 1;
+            hi = next < hi ? static_cast<int>(next) : hi;
+        }
     }
-    *long_row = lo;
+    return lo;
+}
+
+// Entries [e, stop) of a contiguous output range at `out0`, every stride-th
+// one: entry e lies in the last of the `rows` rows whose start is <= e and
+// comes from entry shift[row] + e of the original arrays.
+__device__ __forceinline__ void copy_entries(const int* __restrict__ start,
+                                             const int* __restrict__ shift, int rows, int e,
+                                             int stop, int stride, long long out0,
+                                             const int* __restrict__ ci,
+                                             const float* __restrict__ val,
+                                             int* __restrict__ ci_out, float* __restrict__ val_out)
+{
+    for (; e < stop; e += kCopy * stride) {
+        int c[kCopy];
+        float v[kCopy];
+#pragma unroll
+        for (int k = 0; k < kCopy; ++k) {
+            const int at = e + k * stride;
+            c[k] = 0;
+            v[k] = 0.0f;
+            if (at < stop) {
+                int lo = 0, hi = rows;  // start[lo] <= at < start[hi]
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if (start[mid] <= at) lo = mid;
+                    else hi = mid;
+                }
+                const int s = shift[lo] + at;
+                c[k] = __builtin_nontemporal_load(ci + s);
+                v[k] = __builtin_nontemporal_load(val + s);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kCopy; ++k) {
+            const int at = e + k * stride;
+            if (at < stop) {
+                __builtin_nontemporal_store(c[k], ci_out + out0 + at);
+                __builtin_nontemporal_store(v[k], val_out + out0 + at);
+            }
+        }
+    }
+}
+
+// Rows of at most kWindowMax entries, 64 to a wave.  (A row's entries are
+// fewer than 2^31 and so is every offset; a shift may be negative.)
+__global__ void __launch_bounds__(kBlock)
+gather_windows(const int* __restrict__ rp, const int* __restrict__ ci,
+               const float* __restrict__ val, const int* __restrict__ origin,
+               const int* __restrict__ rp_out, int n, const int* __restrict__ long_row,
+               int* __restrict__ ci_out, float* __restrict__ val_out)
+{
+    __shared__ int s_start[kBlock];
+    __shared__ int s_shift[kBlock];
+    const int lane = threadIdx.x & 63;
+    const int wave0 = threadIdx.x & ~63;
+    const long long r0 = static_cast<long long>(blockIdx.x) * kBlock + wave0;
+    const int last = min(*long_row, n);
+    if (r0 >= last) return;
+    const int rows = static_cast<int>(min(64ll, last - r0));
+    int begin = 0, end = 0, src = 0;
+    if (lane < rows) {
+        begin = rp_out[r0 + lane];
+        end = rp_out[r0 + lane + 1];
+        if (end > begin) src = rp[origin[r0 + lane]];
+    }
+    const int out0 = __builtin_amdgcn_readfirstlane(begin);
+    const int total = __builtin_amdgcn_readlane(end, rows - 1) - out0;
+    s_start[threadIdx.x] = begin - out0;
+    s_shift[threadIdx.x] = src - (begin - out0);
+    // The wave's own LDS: in order in hardware, the fence is the compiler's.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    copy_entries(s_start + wave0, s_shift + wave0, rows, lane, total, 64, out0, ci, val, ci_out,
+                 val_out);
+}
+
+// long_row[0] = the first reordered row with more than kWindowMax entries
+// (n if none): the degrees are sorted ascending, so those rows are a suffix.
+// One wave; also the offsets' leading zero.
+__global__ void __launch_bounds__(64)
+find_long_rows(const unsigned* __restrict__ sorted_deg, int n, int* __restrict__ long_row,
+               int* __restrict__ rp_out)
+{
+    const int r = wave_partition_point(
+        n, [&](int i) { return sorted_deg[i] <= static_cast<unsigned>(kWindowMax); });
+    if (threadIdx.x == 0) {
+        *long_row = r;
+        rp_out[0] = 0;
+    }
 }
 
 // The entries of the long rows [long_row, n), which fill the output range
 // [rp_out[long_row], nnz): block b copies the kLongChunk entries from
-// rp_out[long_row] + b * kLongChunk on, a thread every kBlock-th entry, so a
-// hub row is spread over many blocks and every access is coalesced.  The
-// first row of the block's range is found by binary search; each thread then
-// walks forward row by row.
+// rp_out[long_row] + b * kLongChunk on, so a hub row is spread over many
+// blocks.  The first wave finds the chunk's first row and reads the places of
+// the at most kChunkRows rows that the chunk touches.
 __global__ void __launch_bounds__(kBlock)
 gather_long(const int* __restrict__ rp, const int* __restrict__ ci, const float* __restrict__ val,
             const int* __restrict__ origin, const int* __restrict__ rp_out, int n,
             const int* __restrict__ long_row, int* __restrict__ ci_out, float* __restrict__ val_out)
 {
-    __shared__ int first_row;
+    __shared__ int s_start[kChunkRows];
+    __shared__ int s_shift[kChunkRows];
+    __shared__ int s_rows;
     const int r0 = *long_row;
     if (r0 >= n) return;
     const long long begin = static_cast<long long>(rp_out[r0]) +
                             static_cast<long long>(blockIdx.x) * kLongChunk;
     const long long end = rp_out[n];
     if (begin >= end) return;
-    if (threadIdx.x == 0) {
-        int lo = r0, hi = n - 1;  // last row whose start is <= begin
-        while (lo < hi) {
-            const int mid = hi - (hi - lo) / 2;
-            if (rp_out[mid] <= begin) lo = mid;
-            else hi = mid - 1;
+    const int total = static_cast<int>(min(static_cast<long long>(kLongChunk), end - begin));
+    if (threadIdx.x < 64) {
+        // The last row whose start is <= begin; rows are touched up to the
+        // last one that starts before the chunk's end.
+        const int first =
+            r0 + wave_partition_point(n - r0, [&](int i) { return rp_out[r0 + i] <= begin; }) - 1;
+        int rows = 0;
+        for (int i0 = 0; i0 < kChunkRows; i0 += 64) {
+            const int i = i0 + static_cast<int>(threadIdx.x);
+            const long long row = static_cast<long long>(first) + i;
+            bool in = i < kChunkRows && row < n;
+            if (in) {
+                const long long at = rp_out[row] - begin;  // the row's start in the chunk
+                in = at < total;
+                if (in) {
+                    s_start[i] = static_cast<int>(max(at, 0ll));
+                    s_shift[i] = static_cast<int>(rp[origin[row]] - at);
+                }
+            }
+            rows += __popcll(__ballot(in));
         }
-        first_row = lo;
+        if (threadIdx.x == 0) s_rows = rows;
     }
     __syncthreads();
-    int row = first_row;
-    int row_begin = rp_out[row];
-    int row_end = rp_out[row + 1];
-    int src = rp[origin[row]];
-    const long long stop = min(end, begin + kLongChunk);
-    for (long long p = begin + threadIdx.x; p < stop; p += kBlock) {
-        while (p >= row_end) {
-            ++row;
-            row_begin = row_end;
-            row_end = rp_out[row + 1];
-            src = rp[origin[row]];
-        }
-        const long long s = src + (p - row_begin);
-        ci_out[p] = ci[s];
-        val_out[p] = val[s];
-    }
+    copy_entries(s_start, s_shift, s_rows, threadIdx.x, total, kBlock, begin, ci, val, ci_out,
+                 val_out);
 }
 
 __global__ void set_first_zero(int* __restrict__ p) { p[0] = 0; }
 
-// The two status words of the reorder, cleared by a kernel rather than
-// hipMemsetAsync (memset nodes are kept out of anything a caller may record
-// into a graph).
-__global__ void clear_two(int* __restrict__ p)
-{
-    p[0] = 0;
-    p[1] = 0;
-}
-
-struct DevMem {
-    void* p = nullptr;
-    DevMem() = default;
-    DevMem(const DevMem&) = delete;
-    DevMem& operator=(const DevMem&) = delete;
-    ~DevMem()
-    {
-        if (p) (void)hipFree(p);
-    }
-    hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 1); }
-};
+// The state is cleared by a kernel rather than hipMemsetAsync (memset nodes
+// are kept out of anything a caller may record into a graph).
+__global__ void clear_state(ReorderState* __restrict__ p) { *p = ReorderState{0, 0u, 0, 0}; }
 
 unsigned bits_for(unsigned v)
 {
@@ -207,6 +295,17 @@ cwlb_status grow(T** p, long long have, long long want)
     if (*p) CWLB_HIP_TRY(hipFree(*p));
     *p = nullptr;
     CWLB_HIP_TRY(hipMalloc(reinterpret_cast<void**>(p), sizeof(T) * static_cast<size_t>(want)));
+    return CWLB_OK;
+}
+
+cwlb_status grow_bytes(void** p, size_t* have, size_t want)
+{
+    if (want <= *have && *p) return CWLB_OK;
+    if (*p) CWLB_HIP_TRY(hipFree(*p));
+    *p = nullptr;
+    *have = 0;
+    CWLB_HIP_TRY(hipMalloc(p, want ? want : 1));
+    *have = want;
     return CWLB_OK;
 }
 
@@ -253,13 +352,8 @@ cwlb_status build_run_order(cwlb_ctx* ctx, const SpmmArgs& a, int M, long long n
     size_t bytes = 0;
     CWLB_HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes, ctx->d_run_keys, ctx->d_run_keys_sorted,
                                            ids, ctx->d_run_order, n_runs, 0u, end_bit, st));
-    if (bytes > ctx->sort_temp_bytes || !ctx->d_sort_temp) {
-        if (ctx->d_sort_temp) CWLB_HIP_TRY(hipFree(ctx->d_sort_temp));
-        ctx->d_sort_temp = nullptr;
-        ctx->sort_temp_bytes = 0;
-        CWLB_HIP_TRY(hipMalloc(&ctx->d_sort_temp, bytes ? bytes : 1));
-        ctx->sort_temp_bytes = bytes;
-    }
+    const cwlb_status gs = grow_bytes(&ctx->d_sort_temp, &ctx->sort_temp_bytes, bytes);
+    if (gs != CWLB_OK) return gs;
     const unsigned grid = static_cast<unsigned>((n_runs + kBlock - 1) / kBlock);
     hipLaunchKernelGGL(run_keys, dim3(grid), dim3(kBlock), 0, st, a.tasks,
                        static_cast<long long>(a.n_tasks), M, n_runs, a.origin, a.n_rows,
@@ -299,36 +393,34 @@ cwlb_status launch_reorder(cwlb_ctx* ctx, int32_t n, int64_t nnz, const int32_t*
 
     const size_t un = static_cast<size_t>(n);
     const unsigned grid = static_cast<unsigned>((un + kBlock - 1) / kBlock);
-    DevMem keys, keys_sorted, flags, bmax;
-    CWLB_HIP_TRY(keys.alloc(sizeof(unsigned) * un));
-    CWLB_HIP_TRY(keys_sorted.alloc(sizeof(unsigned) * un));
-    CWLB_HIP_TRY(flags.alloc(2 * sizeof(int)));
-    CWLB_HIP_TRY(bmax.alloc(sizeof(unsigned) * grid));
-    auto* d_keys = static_cast<unsigned*>(keys.p);
-    auto* d_sorted = static_cast<unsigned*>(keys_sorted.p);
-    auto* d_status = static_cast<int*>(flags.p);
-    auto* d_max = reinterpret_cast<unsigned*>(d_status + 1);
-    hipLaunchKernelGGL(clear_two, dim3(1), dim3(1), 0, st, d_status);
-    CWLB_LAUNCH_CHECK("clear_two");
+    // Workspace: the state, the first long row, the block maxima, the keys
+    // and the sorted keys.
+    const size_t b_state = 64;
+    const size_t want = b_state + sizeof(unsigned) * (grid + 2 * un);
+    cwlb_status gs = grow_bytes(&ctx->d_reorder, &ctx->reorder_bytes, want);
+    if (gs != CWLB_OK) return gs;
+    auto* d_state = static_cast<ReorderState*>(ctx->d_reorder);
+    auto* d_long = reinterpret_cast<int*>(d_state + 1);
+    auto* d_keys = reinterpret_cast<unsigned*>(static_cast<char*>(ctx->d_reorder) + b_state);
+    unsigned* d_sorted = d_keys + un;
+    unsigned* d_bmax = d_sorted + un;
+    hipLaunchKernelGGL(clear_state, dim3(1), dim3(1), 0, st, d_state);
+    CWLB_LAUNCH_CHECK("clear_state");
     hipLaunchKernelGGL(degree_keys, dim3(grid), dim3(kBlock), 0, st, rp, n,
-                       static_cast<long long>(nnz), d_keys, d_status,
-                       static_cast<unsigned*>(bmax.p));
+                       static_cast<long long>(nnz), d_keys, &d_state->status, d_bmax);
     CWLB_LAUNCH_CHECK("degree_keys");
-    hipLaunchKernelGGL(reduce_max, dim3(1), dim3(1024), 0, st, static_cast<unsigned*>(bmax.p),
-                       static_cast<long long>(grid), d_max);
+    hipLaunchKernelGGL(reduce_max, dim3(1), dim3(1024), 0, st, d_bmax,
+                       static_cast<long long>(grid), rp, n, d_state);
     CWLB_LAUNCH_CHECK("reduce_max");
-    int host_flags[2] = {0, 0};
-    int ends[2] = {0, 0};
-    CWLB_HIP_TRY(hipMemcpyAsync(host_flags, d_status, sizeof host_flags, hipMemcpyDeviceToHost, st));
-    CWLB_HIP_TRY(hipMemcpyAsync(&ends[0], rp, sizeof(int), hipMemcpyDeviceToHost, st));
-    CWLB_HIP_TRY(hipMemcpyAsync(&ends[1], rp + n, sizeof(int), hipMemcpyDeviceToHost, st));
+    ReorderState state{};
+    CWLB_HIP_TRY(hipMemcpyAsync(&state, d_state, sizeof state, hipMemcpyDeviceToHost, st));
     CWLB_HIP_TRY(hipStreamSynchronize(st));
-    if (host_flags[0] & 1)
+    if (state.status & 1)
         return fail(CWLB_INVALID_ARG, "cwlb_reorder_by_degree_device: row_ptr not a CSR offset array");
-    if (static_cast<int64_t>(ends[1]) - ends[0] != nnz)
+    if (static_cast<int64_t>(state.last) - state.first != nnz)
         return fail(CWLB_RUNTIME_ERROR,
                     "DPL CPU degree reordering produced an inconsistent NNZ count.");
-    const unsigned end_bit = std::max(1u, bits_for(static_cast<unsigned>(host_flags[1])));
+    const unsigned end_bit = std::max(1u, bits_for(state.max_deg));
 
     rocprim::counting_iterator<int> ids(0);
     size_t sort_bytes = 0, scan_bytes = 0;
@@ -336,28 +428,24 @@ cwlb_status launch_reorder(cwlb_ctx* ctx, int32_t n, int64_t nnz, const int32_t*
                                            0u, end_bit, st));
     CWLB_HIP_TRY(rocprim::inclusive_scan(nullptr, scan_bytes, d_sorted, rp_out + 1, un,
                                          rocprim::plus<unsigned>(), st));
-    DevMem temp;
-    CWLB_HIP_TRY(temp.alloc(std::max(sort_bytes, scan_bytes)));
+    gs = grow_bytes(&ctx->d_sort_temp, &ctx->sort_temp_bytes, std::max(sort_bytes, scan_bytes));
+    if (gs != CWLB_OK) return gs;
     size_t bytes = sort_bytes;
-    CWLB_HIP_TRY(rocprim::radix_sort_pairs(temp.p, bytes, d_keys, d_sorted, ids, origin, un, 0u,
-                                           end_bit, st));
+    CWLB_HIP_TRY(rocprim::radix_sort_pairs(ctx->d_sort_temp, bytes, d_keys, d_sorted, ids, origin,
+                                           un, 0u, end_bit, st));
     bytes = scan_bytes;
-    CWLB_HIP_TRY(rocprim::inclusive_scan(temp.p, bytes, d_sorted, rp_out + 1, un,
+    CWLB_HIP_TRY(rocprim::inclusive_scan(ctx->d_sort_temp, bytes, d_sorted, rp_out + 1, un,
                                          rocprim::plus<unsigned>(), st));
-    hipLaunchKernelGGL(set_first_zero, dim3(1), dim3(1), 0, st, rp_out);
-    CWLB_HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(find_long_rows, dim3(1), dim3(64), 0, st, d_sorted, n, d_long, rp_out);
+    CWLB_LAUNCH_CHECK("find_long_rows");
     if (nnz > 0) {
-        hipLaunchKernelGGL(gather_rows, dim3(grid), dim3(kBlock), 0, st, rp, ci, val, origin,
-                           rp_out, n, ci_out, val_out);
-        CWLB_LAUNCH_CHECK("gather_rows");
-        // d_status[0] is free again (checked above): it receives the first
-        // long row.  The long rows hold at most nnz entries.
-        hipLaunchKernelGGL(find_long_rows, dim3(1), dim3(1), 0, st, d_sorted, n, d_status);
-        CWLB_LAUNCH_CHECK("find_long_rows");
+        hipLaunchKernelGGL(gather_windows, dim3(grid), dim3(kBlock), 0, st, rp, ci, val, origin,
+                           rp_out, n, d_long, ci_out, val_out);
+        CWLB_LAUNCH_CHECK("gather_windows");
         const unsigned long_grid =
             static_cast<unsigned>((static_cast<uint64_t>(nnz) + kLongChunk - 1) / kLongChunk);
         hipLaunchKernelGGL(gather_long, dim3(long_grid), dim3(kBlock), 0, st, rp, ci, val,
-                           origin, rp_out, n, d_status, ci_out, val_out);
+                           origin, rp_out, n, d_long, ci_out, val_out);
         CWLB_LAUNCH_CHECK("gather_long");
     }
     CWLB_HIP_TRY(hipStreamSynchronize(st));
