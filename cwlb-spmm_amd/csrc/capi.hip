@@ -306,7 +306,8 @@ cwlb_status cwlb_ctx_destroy(cwlb_ctx* ctx)
                     static_cast<void*>(ctx->d_run_order), ctx->d_sort_temp, ctx->d_part, ctx->d_reorder,
                     static_cast<void*>(ctx->d_col_counts), static_cast<void*>(ctx->d_count_hist),
                     static_cast<void*>(ctx->d_hints), static_cast<void*>(ctx->d_phase_bounds),
-                    static_cast<void*>(ctx->d_band_col), static_cast<void*>(ctx->d_band_val)})
+                    static_cast<void*>(ctx->d_band_col), static_cast<void*>(ctx->d_band_val),
+                    static_cast<void*>(ctx->d_band_h)})
         if (p) (void)hipFree(p);
     for (void* p : ctx->retired) (void)hipFree(p);
     for (int b = 0; b < 2; ++b) {

@@ -96,6 +96,10 @@ struct cwlb_ctx {
     long long band_cap_col = 0;
     float* d_band_val = nullptr;
     long long band_cap_val = 0;
+    // The band-by-band copy of the feature matrix (also rewritten by each
+    // phased call that uses one).
+    float* d_band_h = nullptr;
+    long long band_cap_h = 0;
     int phase_seq = 0;
     cwlb_launch_info last_launch{};  // the last aggregation launch's schedule
     // Pinned host staging of the host-pointer entry point: two buffers used
@@ -194,22 +198,32 @@ struct PhaseArrays {
     int32_t* bounds = nullptr;  // (P - 1) x n_rows
     int32_t* col = nullptr;     // nnz, each row's nonzeros sorted by band
     float* val = nullptr;       // nnz, likewise
+    // The copy of H (null: none), slices x phases x h_rows rows of h_ld
+    // floats; col then holds c / P, the place of column c in its band.
+    float* h = nullptr;
+    int32_t h_ld = 0;
+    int64_t h_rows = 0;
 };
 
 // Sizes the context's phase buffers for `phases` column phases
 // (csrc/col_phases.hip); all null when they cannot be used (a stream under
 // graph capture, where nothing is allocated, and buffers too small).
-cwlb_status prepare_column_phases(cwlb_ctx* ctx, const SpmmArgs& a, int phases, bool may_build,
-                                  PhaseArrays* out);
+cwlb_status prepare_column_phases(cwlb_ctx* ctx, const SpmmArgs& a, int phases, int slices,
+                                  bool may_build, PhaseArrays* out);
+
+// Enqueues the copy of H into out.h for `slices` feature slices.
+cwlb_status launch_band_copy(hipStream_t st, const SpmmArgs& a, int phases, int slices,
+                             const PhaseArrays& out);
 
 // Enqueues the band sort: bounds[(p - 1) * n_rows + r] for p in [1, phases)
 // (bounds may be null) and, when col_out is non-null, the band-sorted copy
 // of col_idx and val.  A non-null chain_word (the aggregation's status[1])
-// is cleared by the same launch.
+// is cleared by the same launch.  places: col_out receives c / P instead of
+// c (INT32_MAX for a column outside [0, h_rows)).
 cwlb_status launch_band_sort(hipStream_t st, const int32_t* row_ptr, const int32_t* col_idx,
                              const float* val, int32_t n_rows, int64_t nnz, int64_t h_rows,
                              int phases, int32_t* bounds, int32_t* col_out, float* val_out,
-                             int32_t* chain_word = nullptr);
+                             int32_t* chain_word = nullptr, bool places = false);
 
 cwlb_status launch_reorder(cwlb_ctx* ctx, int32_t n_rows, int64_t nnz, const int32_t* row_ptr,
                            const int32_t* col_idx, const float* val, int32_t* origin,

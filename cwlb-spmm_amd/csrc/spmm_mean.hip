@@ -421,7 +421,8 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                const unsigned long long* __restrict__ hints, float* __restrict__ C,
                int* __restrict__ status, const int* __restrict__ pb,
                const int* __restrict__ pe, const int* __restrict__ ci_b,
-               const float* __restrict__ val_b, int first_phase, int seq, int write_empty)
+               const float* __restrict__ val_b, const float* __restrict__ hb, int hb_ld,
+               long long hb_rows, long long hb_slice, int first_phase, int seq, int write_empty)
 {
     static_assert(!HN || VEC == 4, "hinted gathers move 16 bytes per lane");
     using V = typename VecT<VEC>::T;
@@ -494,6 +495,18 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                            const int* __restrict__ cx, const float* __restrict__ vx,
                            const bool banded) {
         const bool bph = PH && ph && banded;
+        // The rows gathered: this slice of H or, for the band-sorted copy of
+        // the columns, of the band's copy.
+        const float* __restrict__ Hg = Hs;
+        int ldg = ld;
+        long long rows_g = h_rows;
+        if constexpr (PH) {
+            if (bph && hb) {
+                Hg = hb + slice * hb_slice;
+                ldg = hb_ld;
+                rows_g = hb_rows;
+            }
+        }
         const int rlo = max(rs, 0);
         const int rhi = min(re, n_rows);
         // The staged nonzeros: [st0, st0 + stn) of cx / vx.
@@ -606,7 +619,7 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                                     cold[u] = HN && cc[u] < 0;
                                     if constexpr (HN) cc[u] &= 0x7fffffff;
                                     if (ok[u] && static_cast<unsigned long long>(cc[u]) >=
-                                                     static_cast<unsigned long long>(h_rows)) {
+                                                     static_cast<unsigned long long>(rows_g)) {
                                         ok[u] = false;
                                         bad |= 1;
                                     }
@@ -614,7 +627,7 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                                 V h[UL][R];
 #pragma unroll
                                 for (int u = 0; u < UL; ++u) {
-                                    const float* hrow = Hs + static_cast<size_t>(cc[u]) * ld;
+                                    const float* hrow = Hg + static_cast<size_t>(cc[u]) * ldg;
 #pragma unroll
                                     for (int q = 0; q < R; ++q) {
                                         const int f = fl + G * q;
@@ -750,7 +763,7 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                             cold[u] = HN && cc[u] < 0;
                             if constexpr (HN) cc[u] &= 0x7fffffff;
                             if (ok[u] && static_cast<unsigned long long>(cc[u]) >=
-                                             static_cast<unsigned long long>(h_rows)) {
+                                             static_cast<unsigned long long>(rows_g)) {
                                 ok[u] = false;
                                 bad |= 1;
                             }
@@ -758,7 +771,7 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                         V h[RU][R];
 #pragma unroll
                         for (int u = 0; u < RU; ++u) {
-                            const float* hrow = Hs + static_cast<size_t>(cc[u]) * ld;
+                            const float* hrow = Hg + static_cast<size_t>(cc[u]) * ldg;
 #pragma unroll
                             for (int q = 0; q < R; ++q) {
                                 const int f = fl + G * q;
@@ -1049,6 +1062,10 @@ struct Plan {
     const int* pe;
     const int* cb;    // the band-sorted copy of the columns
     const float* vb;  // and of the values
+    const float* hb;  // the copy of this band's feature rows, or null: their
+    int hb_ld;        // floats per row, rows per band and floats per slice
+    long long hb_rows;
+    long long hb_slice;
     int first;
     int seq;
     int write_empty;  // store rows without nonzeros (as zeros)
@@ -1074,8 +1091,8 @@ int launch_main(hipStream_t st, const SpmmArgs& a, const Plan& p, int* status)
                        a.col_idx, a.val, a.origin, a.n_rows, static_cast<long long>(a.nnz), a.H,
                        static_cast<long long>(a.h_rows), a.K, a.tasks,
                        static_cast<long long>(a.n_tasks), p.M, p.runs, p.blocks, p.chunk, p.order,
-                       p.hints, a.C, status, p.pb, p.pe, p.cb, p.vb, p.first, p.seq,
-                       p.write_empty);
+                       p.hints, a.C, status, p.pb, p.pe, p.cb, p.vb, p.hb, p.hb_ld, p.hb_rows,
+                       p.hb_slice, p.first, p.seq, p.write_empty);
     return waves_per_cu;
 }
 
@@ -1351,6 +1368,10 @@ Plan make_plan(const cwlb_ctx* ctx, const SpmmArgs& a, bool per_task)
     p.pe = nullptr;
     p.cb = nullptr;
     p.vb = nullptr;
+    p.hb = nullptr;
+    p.hb_ld = 0;
+    p.hb_rows = 0;
+    p.hb_slice = 0;
     p.first = 1;
     p.seq = 0;
     p.write_empty = 1;
@@ -1393,7 +1414,7 @@ cwlb_status launch_spmm_mean(cwlb_ctx* ctx, const SpmmArgs& a, bool zero_all, bo
     // one pass, with the same result).
     PhaseArrays ph_arr;
     if (p.phases > 1 && work) {
-        const cwlb_status s = prepare_column_phases(ctx, a, p.phases, may_build, &ph_arr);
+        const cwlb_status s = prepare_column_phases(ctx, a, p.phases, p.sl, may_build, &ph_arr);
         if (s != CWLB_OK) return s;
     }
     if (!ph_arr.bounds) p.phases = 1;
@@ -1450,8 +1471,16 @@ cwlb_status launch_spmm_mean(cwlb_ctx* ctx, const SpmmArgs& a, bool zero_all, bo
     if (p.phases > 1) {
         const cwlb_status s =
             launch_band_sort(st, a.row_ptr, a.col_idx, a.val, a.n_rows, a.nnz, a.h_rows,
-                             p.phases, ph_arr.bounds, ph_arr.col, ph_arr.val, ctx->d_status + 1);
+                             p.phases, ph_arr.bounds, ph_arr.col, ph_arr.val, ctx->d_status + 1,
+                             ph_arr.h != nullptr);
         if (s != CWLB_OK) return s;
+        if (ph_arr.h) {
+            const cwlb_status c = launch_band_copy(st, a, p.phases, p.sl, ph_arr);
+            if (c != CWLB_OK) return c;
+            p.hb_ld = ph_arr.h_ld;
+            p.hb_rows = ph_arr.h_rows;
+            p.hb_slice = ph_arr.h_rows * p.phases * ph_arr.h_ld;
+        }
     }
     if ((!zero_all || p.phases > 1) && work) {
         if (p.vec == 4) launch_zero<4>(st, a, p, ctx->d_status);
@@ -1472,6 +1501,7 @@ cwlb_status launch_spmm_mean(cwlb_ctx* ctx, const SpmmArgs& a, bool zero_all, bo
             const long long n = a.n_rows;
             p.pb = ph > 0 ? ph_arr.bounds + (ph - 1) * n : nullptr;
             p.pe = ph < p.phases - 1 ? ph_arr.bounds + ph * n : nullptr;
+            if (ph_arr.h) p.hb = ph_arr.h + ph * ph_arr.h_rows * ph_arr.h_ld;
             p.first = ph == 0;
             if (p.vec == 4) waves = dispatch_main<4>(st, a, p, ctx->d_status);
             else if (p.vec == 2) waves = dispatch_main<2>(st, a, p, ctx->d_status);

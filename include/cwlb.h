@@ -194,9 +194,12 @@ cwlb_status cwlb_ctx_get_lane_tiling(cwlb_ctx* ctx, int32_t* tiling);
  * phased call first writes, into context-owned buffers, a copy of col_idx
  * and val with every row's nonzeros stably sorted by band and the row
  * bounds of the bands (see cwlb_column_phase_sort; 8 bytes per nonzero
- * and 4 (P - 1) per row, kept and grown as needed; about 0.3 ms on a
- * 115M-nonzero graph, reported in the timing's zero_us), so rewritten
- * arrays are always read as they are.  A row that one stretch of
+ * and 4 (P - 1) per row, kept and grown as needed) and, where feature slices
+ * are not whole 128-byte lines, H holds at least 32 MB and 32 nonzeros per
+ * feature row, a copy of H with padded slices (about the size of H; left out
+ * where there is no memory for it).  On a 115M-nonzero graph at K = 600
+ * this takes 0.8 ms, reported in the timing's zero_us; rewritten arrays are
+ * always read as they are.  A row that one stretch of
  * consecutive tasks covers whole (see CWLB_SPMM_PER_TASK) is stored in the
  * first pass and added to in the others without atomics, which reads and
  * writes C P times: phases pay when H is well beyond the 256 MB Infinity
