@@ -106,15 +106,19 @@ struct VecT<4> {
 };
 
 
+// 16 bytes at any 4-byte boundary, for rows that are not whole vectors.
+typedef f4 f4u __attribute__((aligned(4)));
+
 template <int VEC>
 __device__ __forceinline__ typename VecT<VEC>::T vzero()
 {
     return typename VecT<VEC>::T(0.0f);
 }
 
-template <int VEC>
+template <int VEC, bool RG = false>
 __device__ __forceinline__ typename VecT<VEC>::T vload(const float* p)
 {
+    if constexpr (RG) return *reinterpret_cast<const f4u*>(p);
     return *reinterpret_cast<const typename VecT<VEC>::T*>(p);
 }
 
@@ -125,9 +129,13 @@ __device__ __forceinline__ void vstore(float* p, typename VecT<VEC>::T v)
 }
 
 // Streaming (non-temporal) store: C is written once and not re-read.
-template <int VEC>
+template <int VEC, bool RG = false>
 __device__ __forceinline__ void vstore_nt(float* p, typename VecT<VEC>::T v)
 {
+    if constexpr (RG) {
+        __builtin_nontemporal_store(v, reinterpret_cast<f4u*>(p));
+        return;
+    }
     __builtin_nontemporal_store(v, reinterpret_cast<typename VecT<VEC>::T*>(p));
 }
 
@@ -162,13 +170,6 @@ __device__ __forceinline__ int with_hint(int col, const unsigned long long* __re
 }
 
 __device__ __forceinline__ float vfma(float a, float h, float c) { return __builtin_fmaf(a, h, c); }
-__device__ __forceinline__ f2 vfma(float a, f2 h, f2 c)
-{
-    f2 r;
-    r.x = __builtin_fmaf(a, h.x, c.x);
-    r.y = __builtin_fmaf(a, h.y, c.y);
-    return r;
-}
 __device__ __forceinline__ f4 vfma(float a, f4 h, f4 c)
 {
     f4 r;
@@ -180,13 +181,6 @@ __device__ __forceinline__ f4 vfma(float a, f4 h, f4 c)
 }
 
 __device__ __forceinline__ float vdiv(float v, float d) { return v / d; }
-__device__ __forceinline__ f2 vdiv(f2 v, float d)
-{
-    f2 r;
-    r.x = v.x / d;
-    r.y = v.y / d;
-    return r;
-}
 __device__ __forceinline__ f4 vdiv(f4 v, float d)
 {
     f4 r;
@@ -197,14 +191,14 @@ __device__ __forceinline__ f4 vdiv(f4 v, float d)
     return r;
 }
 
-__device__ __forceinline__ float vshfl_xor(float v, int m) { return __shfl_xor(v, m); }
-__device__ __forceinline__ f2 vshfl_xor(f2 v, int m)
+// Float i of a vector.
+__device__ __forceinline__ float component(float v, int) { return v; }
+__device__ __forceinline__ float component(f4 v, int i)
 {
-    f2 r;
-    r.x = __shfl_xor(v.x, m);
-    r.y = __shfl_xor(v.y, m);
-    return r;
+    return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
 }
+
+__device__ __forceinline__ float vshfl_xor(float v, int m) { return __shfl_xor(v, m); }
 __device__ __forceinline__ f4 vshfl_xor(f4 v, int m)
 {
     f4 r;
@@ -216,11 +210,6 @@ __device__ __forceinline__ f4 vshfl_xor(f4 v, int m)
 }
 
 __device__ __forceinline__ void vatomic_add(float* p, float v) { unsafeAtomicAdd(p, v); }
-__device__ __forceinline__ void vatomic_add(float* p, f2 v)
-{
-    unsafeAtomicAdd(p, v.x);
-    unsafeAtomicAdd(p + 1, v.y);
-}
 __device__ __forceinline__ void vatomic_add(float* p, f4 v)
 {
     unsafeAtomicAdd(p, v.x);
@@ -241,9 +230,21 @@ __device__ __forceinline__ int write_mode(bool ph, bool first, const Ch& c)
     return (c.b == 0 && c.e == c.d) ? 0 : 2;
 }
 
-template <int VEC>
-__device__ __forceinline__ void write_row(float* p, typename VecT<VEC>::T v, int how)
+// (RG: the first `skip` floats of the vector belong to the lane before, which
+// stores the same values but must alone add them.)
+template <int VEC, bool RG>
+__device__ __forceinline__ void write_row(float* p, typename VecT<VEC>::T v, int how, int skip)
 {
+    if constexpr (RG) {
+        if (how == 0) {
+            vstore_nt<VEC, RG>(p, v);
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < VEC; ++i)
+            if (i >= skip) vatomic_add(p + i, v[i]);
+        return;
+    }
     if (how == 0)
         vstore_nt<VEC>(p, v);
     else if (how == 1)
@@ -411,7 +412,7 @@ __device__ __forceinline__ void block_slice(int& slice, long long& jb, long long
 // over ci / val in the first launch and not at all in the others).
 // write_empty: rows without nonzeros are stored as zeros; 0 leaves them to
 // the caller's clearing, as the reference's kernel never writes them.
-template <int VEC, int G, int R, int U, int SL, bool HN, bool O6, bool PH>
+template <int VEC, int G, int R, int U, int SL, bool HN, bool O6, bool PH, bool RG>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(O6 ? 6 : 1)))
 spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                const float* __restrict__ val, const int* __restrict__ origin, int n_rows,
@@ -425,6 +426,7 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                long long hb_rows, long long hb_slice, int first_phase, int seq, int write_empty)
 {
     static_assert(!HN || VEC == 4, "hinted gathers move 16 bytes per lane");
+    static_assert(!RG || (VEC == 4 && SL == 1 && !HN && !PH), "ragged rows: the plain kernel");
     using V = typename VecT<VEC>::T;
     constexpr int NS = 64 / G;                     // row slots per wave
     constexpr int RU = cmin(cmin(U, 4), G);        // rows per slot (short rows)
@@ -476,7 +478,11 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
 
     // This slice's vectors [f0, f0 + F) of the row's ld / VEC: whole
     // vectors, as even as the row allows (sizes differ by at most one).
-    const int FT = ld / VEC;
+    // Ragged rows (RG, ld >= 4) have a last vector that ends with the row and
+    // overlaps the one before.
+    const int FT = RG ? (ld + VEC - 1) / VEC : ld / VEC;
+    const int tail = ld - VEC;
+    auto at_vec = [tail](int f) { return RG ? min(f * VEC, tail) : f * VEC; };
     const int f0 = slice * FT / SL;
     const int F = (slice + 1) * FT / SL - f0;
     const float* __restrict__ Hs = H + f0 * VEC;
@@ -573,7 +579,11 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                     }
                     const int cb = c.base + c.b;
                     const int ce = c.base + c.e;
-                    longm = __ballot(c.e - c.b >= kLong);
+                    // Where the run holds few rows, a chunk runs on all slots
+                    // from RU nonzeros per row of the window on: the group
+                    // would take more round trips than the chunks one by one
+                    // (the same graph and width: 32.3 us without, 29.0 with).
+                    longm = __ballot(c.e - c.b >= min(kLong, RU * wcnt + 1));
                     some = __ballot(c.e > c.b);
                     live = some | __ballot(how != 3);
                     last_end = __builtin_amdgcn_readlane(ce, wcnt - 1);
@@ -639,7 +649,7 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                                                                           cold[u])
                                                           : vzero<VEC>();
                                         else
-                                            h[u][q] = (ok[u] && f < F) ? vload<VEC>(hrow + f * VEC)
+                                            h[u][q] = (ok[u] && f < F) ? vload<VEC, RG>(hrow + at_vec(f))
                                                                        : vzero<VEC>();
                                     }
                                 }
@@ -660,14 +670,38 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                             for (int q = 0; q < R; ++q) acc[q] = acc[q] + vshfl_xor(acc[q], off);
                         }
                         const int how = __builtin_amdgcn_readfirstlane(whow[w]);
-                        if (how != 3 && slot == 0) {
+                        if (how != 3) {
                             const int o = __builtin_amdgcn_readfirstlane(wout[w]);
                             float* crow = Cs + static_cast<size_t>(o) * ld;
                             const float fd = wdeg[w];
+                            if (VEC == 4 && NS > 1 && how == 2) {
+                                // Every slot holds the sums: up to four
+                                // share the floats of each vector, a
+                                // quarter of the atomic instructions (20k-row
+                                // power law, K = 50, one task per wave: 29.0
+                                // us with one slot's lanes, 19.7 so).
+                                constexpr int CS = NS < 4 ? NS : 4;
+                                if (slot < CS) {
 #pragma unroll
-                            for (int q = 0; q < R; ++q) {
-                                const int f = fl + G * q;
-                                if (f < F) write_row<VEC>(crow + f * VEC, vdiv(acc[q], fd), how);
+                                    for (int q = 0; q < R; ++q) {
+                                        const int f = fl + G * q;
+#pragma unroll
+                                        for (int t = 0; t < VEC; t += CS) {
+                                            const int i = slot + t;
+                                            if (f < F && i >= f * VEC - at_vec(f))
+                                                vatomic_add(crow + at_vec(f) + i,
+                                                            component(acc[q], i) / fd);
+                                        }
+                                    }
+                                }
+                            } else if (slot == 0) {
+#pragma unroll
+                                for (int q = 0; q < R; ++q) {
+                                    const int f = fl + G * q;
+                                    if (f < F)
+                                        write_row<VEC, RG>(crow + at_vec(f), vdiv(acc[q], fd), how,
+                                                           f * VEC - at_vec(f));
+                                }
                             }
                         }
                         continue;
@@ -694,7 +728,7 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
 #pragma unroll
                                     for (int q = 0; q < R; ++q) {
                                         const int f = fl + G * q;
-                                        if (f < F) vstore_nt<VEC>(crow + f * VEC, vzero<VEC>());
+                                        if (f < F) vstore_nt<VEC, RG>(crow + at_vec(f), vzero<VEC>());
                                     }
                                 }
                             }
@@ -783,7 +817,7 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                                                                   cold[u])
                                                   : vzero<VEC>();
                                 else
-                                    h[u][q] = (ok[u] && f < F) ? vload<VEC>(hrow + f * VEC)
+                                    h[u][q] = (ok[u] && f < F) ? vload<VEC, RG>(hrow + at_vec(f))
                                                                : vzero<VEC>();
                             }
                         }
@@ -824,7 +858,8 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                             for (int q = 0; q < R; ++q) {
                                 const int f = fl + G * q;
                                 if (f < F)
-                                    write_row<VEC>(crow + f * VEC, vdiv(acc[u][q], fd[u]), how[u]);
+                                    write_row<VEC, RG>(crow + at_vec(f), vdiv(acc[u][q], fd[u]), how[u],
+                                                       f * VEC - at_vec(f));
                             }
                         }
                     }
@@ -1041,7 +1076,8 @@ unsigned long long host_mix64(unsigned long long z)
 
 // Launch geometry of one call: M tasks per wave, SL feature slices.
 struct Plan {
-    int vec;
+    int vec;               // floats of a whole vector that rows are made of
+    bool ragged;           // 16-byte lanes all the same (see pick_ragged)
     int sl;
     int M;
     long long runs;
@@ -1073,7 +1109,8 @@ struct Plan {
 
 // Launches one instantiation; returns its resident waves per CU at most
 // (from its register and LDS use, queried once per instantiation).
-template <int VEC, int G, int R, int SL, bool HN = false, bool O6 = false, bool PH = false>
+template <int VEC, int G, int R, int SL, bool HN = false, bool O6 = false, bool PH = false,
+          bool RG = false>
 int launch_main(hipStream_t st, const SpmmArgs& a, const Plan& p, int* status)
 {
     constexpr int U = (R == 1) ? 8 : (R == 2) ? 4 : (R <= 4) ? 2 : 1;
@@ -1081,12 +1118,12 @@ int launch_main(hipStream_t st, const SpmmArgs& a, const Plan& p, int* status)
         int blocks = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
                 &blocks,
-                reinterpret_cast<const void*>(&spmm_mean_runs<VEC, G, R, U, SL, HN, O6, PH>),
+                reinterpret_cast<const void*>(&spmm_mean_runs<VEC, G, R, U, SL, HN, O6, PH, RG>),
                 kBlock, 0) != hipSuccess)
             blocks = 0;
         return blocks * kWaves;
     }();
-    hipLaunchKernelGGL((spmm_mean_runs<VEC, G, R, U, SL, HN, O6, PH>),
+    hipLaunchKernelGGL((spmm_mean_runs<VEC, G, R, U, SL, HN, O6, PH, RG>),
                        dim3(static_cast<unsigned>(p.grid)), dim3(kBlock), 0, st, a.row_ptr,
                        a.col_idx, a.val, a.origin, a.n_rows, static_cast<long long>(a.nnz), a.H,
                        static_cast<long long>(a.h_rows), a.K, a.tasks,
@@ -1217,6 +1254,32 @@ int dispatch_width(hipStream_t st, const SpmmArgs& a, const Plan& p, int* status
     }
 }
 
+// Ragged rows: 16-byte lanes at 4-byte alignment, ceil(K / 4) vectors.
+int dispatch_ragged(hipStream_t st, const SpmmArgs& a, const Plan& p, int* status)
+{
+    const int F = (a.K + 3) / 4;
+    int G = 2;
+    while (G < F && G < 64) G <<= 1;
+    switch (G < 64 ? 0 : std::min((F + 63) / 64, 8)) {
+    case 0:
+        switch (G) {
+        case 2: return launch_main<4, 2, 1, 1, false, false, false, true>(st, a, p, status);
+        case 4: return launch_main<4, 4, 1, 1, false, false, false, true>(st, a, p, status);
+        case 8: return launch_main<4, 8, 1, 1, false, false, false, true>(st, a, p, status);
+        case 16: return launch_main<4, 16, 1, 1, false, false, false, true>(st, a, p, status);
+        default: return launch_main<4, 32, 1, 1, false, false, false, true>(st, a, p, status);
+        }
+    case 1: return launch_main<4, 64, 1, 1, false, false, false, true>(st, a, p, status);
+    case 2: return launch_main<4, 64, 2, 1, false, false, false, true>(st, a, p, status);
+    case 3: return launch_main<4, 64, 3, 1, false, false, false, true>(st, a, p, status);
+    case 4: return launch_main<4, 64, 4, 1, false, false, false, true>(st, a, p, status);
+    case 5: return launch_main<4, 64, 5, 1, false, false, false, true>(st, a, p, status);
+    case 6: return launch_main<4, 64, 6, 1, false, false, false, true>(st, a, p, status);
+    case 7: return launch_main<4, 64, 7, 1, false, false, false, true>(st, a, p, status);
+    default: return launch_main<4, 64, 8, 1, false, false, false, true>(st, a, p, status);
+    }
+}
+
 template <int VEC>
 int dispatch_main(hipStream_t st, const SpmmArgs& a, const Plan& p, int* status)
 {
@@ -1243,6 +1306,20 @@ int pick_vec(const SpmmArgs& a)
     if (a.K % 4 == 0 && h % 16 == 0 && c % 16 == 0) return 4;
     if (a.K % 2 == 0 && h % 8 == 0 && c % 8 == 0) return 2;
     return 1;
+}
+
+// Rows of other widths or alignments move 16 bytes per lane too, at 4-byte
+// boundaries (global loads and stores need no more), the last vector of a row
+// overlapping the one before: K = 75 takes 19 lanes of one load instead of 64
+// lanes of two, and two rows to a wave instead of one (2^18-row R-MAT:
+// 206 us with single floats, 141 us so; 20k-row power law at K = 50, 8-byte
+// lanes before: 24.7 us, 19.7).
+// Rows shorter than a vector, and arrays that are not even 4-byte aligned,
+// stay with single floats.
+bool pick_ragged(const SpmmArgs& a, int vec)
+{
+    const auto at = reinterpret_cast<uintptr_t>(a.H) | reinterpret_cast<uintptr_t>(a.C);
+    return vec != 4 && a.K >= 4 && at % 4 == 0;
 }
 
 // The slot tiling of a slice of F vectors: G lanes per slot, R vectors per
@@ -1314,6 +1391,7 @@ Plan make_plan(const cwlb_ctx* ctx, const SpmmArgs& a, bool per_task)
 {
     Plan p{};
     p.vec = pick_vec(a);
+    p.ragged = pick_ragged(a, p.vec);
     p.M = 1;
     p.sl = 1;
     if (!per_task) {
@@ -1504,8 +1582,8 @@ cwlb_status launch_spmm_mean(cwlb_ctx* ctx, const SpmmArgs& a, bool zero_all, bo
             if (ph_arr.h) p.hb = ph_arr.h + ph * ph_arr.h_rows * ph_arr.h_ld;
             p.first = ph == 0;
             if (p.vec == 4) waves = dispatch_main<4>(st, a, p, ctx->d_status);
-            else if (p.vec == 2) waves = dispatch_main<2>(st, a, p, ctx->d_status);
-            else waves = dispatch_main<1>(st, a, p, ctx->d_status);
+            else if (p.ragged) waves = dispatch_ragged(st, a, p, ctx->d_status);
+            else waves = dispatch_width<1, 1>(st, a, p, ctx->d_status);
             CWLB_HIP_TRY(hipGetLastError());
         }
         ctx->last_launch.max_waves_per_cu = waves;

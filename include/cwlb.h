@@ -249,7 +249,11 @@ typedef struct cwlb_launch_info {
     int32_t run_order;       /* 1 task order, 2 sorted by output row */
     int32_t xcd_blocks;      /* 1 interleaved over the XCDs, 2 contiguous */
     int32_t cache_hints;     /* 1 when the gathers carried cache hints */
-    int32_t vector_width;    /* floats per load: 4, 2 or 1 */
+    int32_t vector_width;    /* floats of the widest vector that rows are made
+                                of and aligned to: 4, 2 or 1.  Rows of 4
+                                floats or more move in 16-byte lanes all the
+                                same; slot_lanes and lane_vectors are those
+                                of lanes of vector_width floats. */
     int32_t waves_per_simd;  /* 6 for the occupancy variant, else 0 */
     int32_t max_waves_per_cu; /* resident waves per CU the kernel's register
                                  and LDS use allow */

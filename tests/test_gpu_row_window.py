@@ -46,7 +46,7 @@ def graph(name):
     return custom_graph(rp, ci, 1.0 - rng.random(len(ci), dtype=np.float32)), h_rows
 
 
-@pytest.mark.parametrize("K", [1, 2, 3, 4, 18, 32, 50, 75, 96, 128, 257, 600, 1028])
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 5, 6, 7, 18, 32, 50, 75, 96, 128, 253, 257, 600, 1027, 1028, 2050])
 @pytest.mark.parametrize("name", list(DEGREES))
 def test_window_edges(gpu_ctx, name, K):
     g, h_rows = graph(name)
