@@ -413,7 +413,7 @@ __device__ __forceinline__ void block_slice(int& slice, long long& jb, long long
 // write_empty: rows without nonzeros are stored as zeros; 0 leaves them to
 // the caller's clearing, as the reference's kernel never writes them.
 template <int VEC, int G, int R, int U, int SL, bool HN, bool O6, bool PH, bool RG>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(O6 ? 6 : 1)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(O6 ? 6 : PH && R == 5 ? 7 : 1)))
 spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                const float* __restrict__ val, const int* __restrict__ origin, int n_rows,
                long long nnz, const float* __restrict__ H, long long h_rows, int ld,
@@ -443,6 +443,7 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
     __shared__ int s_out[kWaves * 64];
     __shared__ float s_deg[kWaves * 64];
     __shared__ int s_how[kWaves * 64];
+    __shared__ int s_src[PH ? kWaves * 64 : 1];  // column phases: see below
     __shared__ int s_col[kWaves * kStage];
     __shared__ float s_val[kWaves * kStage];
 
@@ -456,20 +457,13 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long long pos = jb * kWaves + wv;
     if (pos >= n_runs) return;
-    // Column phases apply to chains only: rows whose whole range one
-    // segment covers are then stored in the first phase and added to,
-    // without atomics, in the others.
-    bool ph = false;
     const bool first = !PH || first_phase != 0;
-    if constexpr (PH) {
-        ph = __builtin_amdgcn_readfirstlane(status[1]) != seq;
-        if (!ph && !first) return;
-    }
     int* const wbeg = s_beg + wv * 64;
     int* const wend = s_end + wv * 64;
     int* const wout = s_out + wv * 64;
     float* const wdeg = s_deg + wv * 64;
     int* const whow = s_how + wv * 64;
+    int* const wsrc = s_src + (PH ? wv * 64 : 0);
     int* const wcol = s_col + wv * kStage;
     float* const wval = s_val + wv * kStage;
     // run_order (optional) is a permutation of [0, n_runs): runs execute in
@@ -493,6 +487,22 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
     __amdgpu_buffer_rsrc_t hrsrc;
     if constexpr (HN) hrsrc = feature_rsrc(H, h_rows, ld);
     const unsigned slice_bytes = static_cast<unsigned>(f0 * VEC) * 4u;
+
+    // Column phases apply to chains only: rows whose whole range one
+    // segment covers are then stored in the first phase and added to,
+    // without atomics, in the others.  The run's tasks are read along with
+    // the word that says so, in one round trip.
+    bool ph = false;
+    const long long t0 = run * M;
+    const int cnt = static_cast<int>(min(static_cast<long long>(M), n_tasks - t0));
+    cwlb_task head_task{0, 0, 0, 0}, tail_task{0, 0, 0, 0}, last_task{0, 0, 0, 0};
+    if constexpr (PH) {
+        head_task = tasks[t0];
+        tail_task = tasks[t0 + cnt - 1];
+        last_task = tasks[n_tasks - 1];
+        ph = __builtin_amdgcn_readfirstlane(status[1]) != seq;
+        if (!ph && !first) return;
+    }
 
     // One segment: task (rs, re, fo, ln) over the column and value arrays
     // cx / vx; banded: the rows are whole rows of a chain, read band by band
@@ -529,8 +539,20 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 const int i = lane + 64 * t;
-                lc[t] = i < n ? __builtin_nontemporal_load(cx + from + i) : 0;
-                lv[t] = i < n ? __builtin_nontemporal_load(vx + from + i) : 0.0f;
+                int at = from + i;
+                if constexpr (PH) {
+                    // The last row that starts at or before nonzero `at` of
+                    // the window (rows past it start at its end).
+                    if (bph && i < n) {
+                        int lo = 0;
+#pragma unroll
+                        for (int half = 32; half > 0; half >>= 1)
+                            if (wbeg[lo + half] <= at) lo += half;
+                        at += wsrc[lo];
+                    }
+                }
+                lc[t] = i < n ? __builtin_nontemporal_load(cx + at) : 0;
+                lv[t] = i < n ? __builtin_nontemporal_load(vx + at) : 0.0f;
                 if constexpr (HN)
                     if (i < n) lc[t] = with_hint(lc[t], hints, from + i);
             }
@@ -577,8 +599,32 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                             how = write_mode<PH>(bph, first, c);
                         }
                     }
-                    const int cb = c.base + c.b;
-                    const int ce = c.base + c.e;
+                    int cb = c.base + c.b;
+                    int ce = c.base + c.e;
+                    int shift = 0;
+                    if constexpr (PH) {
+                        if (bph) {
+                            // A band's chunks are not neighbours in memory:
+                            // the window counts its nonzeros from 0, and a
+                            // row's shift leads to where they are, so that
+                            // one stage holds many rows' chunks (staged row
+                            // by row: 240k-row block model, K = 100, 24
+                            // nonzeros per row, 16 phases, 7.5 ms per call;
+                            // so 1.9 ms.  480 nonzeros per row, K = 600:
+                            // 24.8 and 24.5 ms).
+                            const int len = ce - cb;
+                            int sum = len;
+#pragma unroll
+                            for (int off = 1; off < 64; off <<= 1) {
+                                const int t = __shfl_up(sum, off);
+                                if (lane >= off) sum += t;
+                            }
+                            shift = cb - (sum - len);
+                            cb = sum - len;
+                            ce = sum;
+                            stn = 0;
+                        }
+                    }
                     // Where the run holds few rows, a chunk runs on all slots
                     // from RU nonzeros per row of the window on: the group
                     // would take more round trips than the chunks one by one
@@ -588,6 +634,7 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                     live = some | __ballot(how != 3);
                     last_end = __builtin_amdgcn_readlane(ce, wcnt - 1);
                     wave_lds_fence();
+                    if constexpr (PH) wsrc[lane] = shift;
                     wbeg[lane] = cb;
                     wend[lane] = ce;
                     wout[lane] = o;
@@ -610,7 +657,7 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                             // is left of it, or a whole stage of its own.
                             if (at < st0 || at - st0 >= stn ||
                                 (ce - st0 > stn && at != st0))
-                                stage(at, bph ? ce : max(last_end, ce));
+                                stage(at, max(last_end, ce));
                             const int off = at - st0;
                             const int wn = min(stn - off, ce - at);
                             for (int k0 = 0; k0 < wn; k0 += STEP) {
@@ -754,7 +801,7 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
                         const int fb = __builtin_amdgcn_readfirstlane(b);
                         const int fe = __builtin_amdgcn_readfirstlane(e);
                         if (fb < st0 || fb - st0 >= stn || fe - st0 > stn)
-                            stage(fb, bph ? fe : max(last_end, fe));
+                            stage(fb, max(last_end, fe));
                         const bool fits = lane < upto &&
                                           (e <= b || (b >= st0 && b - st0 < stn && e - st0 <= stn));
                         const unsigned long long stop = __ballot(!fits);
@@ -871,8 +918,6 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
     // The run's tasks, 64 at a time: the window's segment starts by ballot
     // (one coalesced load of the window), then the segments in order, each
     // reading its first and last task.
-    const long long t0 = run * M;
-    const int cnt = static_cast<int>(min(static_cast<long long>(M), n_tasks - t0));
     if constexpr (PH) {
         if (ph) {
             // A chain under column phases: the run takes, whole, every row
@@ -881,9 +926,9 @@ spmm_mean_runs(const int* __restrict__ rp, const int* __restrict__ ci,
             // earlier) to its last task's row, completed -- so each row has
             // one wave and no atomics.  The chain's ends keep their offsets:
             // the first task's start, and the last task's end in its row.
-            const cwlb_task a = tasks[t0];
-            const cwlb_task z = tasks[t0 + cnt - 1];
-            const cwlb_task zl = tasks[n_tasks - 1];
+            const cwlb_task& a = head_task;
+            const cwlb_task& z = tail_task;
+            const cwlb_task& zl = last_task;
             const bool head = t0 == 0;
             const int rs = (head || a.first_row_offset == 0) ? a.row_start : a.row_start + 1;
             const int re = z.row_end;
