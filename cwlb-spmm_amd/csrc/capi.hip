@@ -118,7 +118,7 @@ cwlb_status run_spmm(cwlb_ctx* ctx, const SpmmArgs& a, uint32_t flags, cwlb_timi
 // Host-pointer transfers through the context's two pinned staging buffers:
 // while the DMA engine moves one buffer, the host threads fill (or drain)
 // the other.
-constexpr size_t kStageBytes = size_t{64} << 20;
+constexpr size_t kStageBytes = size_t{32} << 20;
 
 // True when both staging buffers and their events exist (allocated at the
 // first call).  Without them (pinned memory refused) the caller copies

@@ -14,14 +14,14 @@
 
 namespace cwlb {
 
-// fn(begin, end) over [0, n) split into contiguous parts, on up to 8 host
+// fn(begin, end) over [0, n) split into contiguous parts, on up to 16 host
 // threads (about one per `grain` items), the caller's thread included.  The
 // parts are disjoint and every thread is joined before the call returns.
 template <class Fn>
 void parallel_ranges(size_t n, size_t grain, Fn fn)
 {
     const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-    const size_t T = std::max<size_t>(1, std::min<size_t>({size_t{8}, hw, n / grain}));
+    const size_t T = std::max<size_t>(1, std::min<size_t>({size_t{16}, hw, n / grain}));
     if (T == 1) {
         fn(size_t{0}, n);
         return;
@@ -34,10 +34,10 @@ void parallel_ranges(size_t n, size_t grain, Fn fn)
     for (auto& th : pool) th.join();
 }
 
-// memcpy of `bytes` bytes in parts of about 8 MiB on up to 8 threads.
+// memcpy of `bytes` bytes in parts of about 2 MiB on up to 16 threads.
 inline void parallel_copy(void* dst, const void* src, size_t bytes)
 {
-    parallel_ranges(bytes, size_t{8} << 20, [&](size_t b, size_t e) {
+    parallel_ranges(bytes, size_t{2} << 20, [&](size_t b, size_t e) {
         std::memcpy(static_cast<char*>(dst) + b, static_cast<const char*>(src) + b, e - b);
     });
 }
