@@ -28,11 +28,12 @@
 //      the chain from the block's entry node; each marked node simulates
 //      again and writes its tasks; rows of 64 segments or more are set aside;
 //   6. part_segments: a wave writes the tasks of such a row.
-// Nothing is written when the total exceeds the caller's buffer.  The host waits once, for the total and the status.  Measured on the
-// 4.2M-row R-MAT graph (1.08M tasks): 12.7 ms per call when the doubling ran
-// over all nodes of the graph in global memory (23 jump tables, 413 MB
-// allocated and freed by the call), 345 us now (part_emit 190, part_blocks 58,
-// part_walk 35, part_groups 17, part_check 6, part_segments 6).
+// Nothing is written when the total exceeds the caller's buffer.  The host
+// waits once, for the total and the status.  Measured on the 4.2M-row R-MAT
+// graph (1.08M tasks): 12.7 ms per call when the doubling ran over all nodes
+// of the graph in global memory (23 jump tables, 413 MB allocated and freed
+// by the call), 345 us now (part_emit 190, part_blocks 58, part_walk 35,
+// part_groups 17, part_check 6, part_segments 6).
 // Node ids: A(r) = 2 r for r in [0, n] (A(n) is the end), B(r) = 2 r + 1.
 //
 // A short-row scan adds at least C_store per row, so it is bounded by
@@ -428,8 +429,8 @@ part_emit(PartParams p, Layout l, SetAside* __restrict__ aside, cwlb_task* __res
 }
 
 // The rows set aside, a wave each: the hub rows are neighbours in the order,
-// and one work-group alone writes 16-byte tasks no faster than 30 GB/s (the
-// R-MAT graph's last block: 160 us).
+// so that a few work-groups would write most of the tasks (R-MAT: part_emit
+// 218 us with its own waves doing this, 203 us and 6 us here without).
 __global__ void __launch_bounds__(kBlock)
 part_segments(int S, const PartState* __restrict__ st, const SetAside* __restrict__ aside,
               cwlb_task* __restrict__ out)
