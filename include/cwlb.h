@@ -402,9 +402,9 @@ cwlb_status cwlb_ctx_tune_schedule(cwlb_ctx* ctx, const int32_t* row_ptr, const 
  * like run_single_s (main.cpp:359-365).  A task list that does not tile the
  * nonzeros in order runs one task per wave, so every list, overlapping ones
  * included, gives the reference's result.  Timing covers the kernels only.
- * The host arrays may be pageable: transfers go through two 64 MiB pinned
+ * The host arrays may be pageable: transfers go through two 32 MiB pinned
  * staging buffers that the context allocates at its first host-pointer call
- * and keeps until cwlb_ctx_destroy, filled and drained by up to 8 host
+ * and keeps until cwlb_ctx_destroy, filled and drained by up to 16 host
  * threads while the DMA engine moves the other buffer (if pinned memory is
  * refused, the arrays are copied directly). */
 cwlb_status cwlb_spmm_mean_f32_host(cwlb_ctx* ctx, const int32_t* row_ptr,
